@@ -226,7 +226,7 @@ inline ProgramInputs program_inputs(const qr::Engine &eng)
 
 struct DevTables
 {
-    DevBuf srf, mat, lgt, clp, elem, tex, step, step_any, refit_in, refit_box;
+    DevBuf srf, hot, mat, lgt, clp, elem, tex, step, step_any, refit_in, refit_box;
     DevBuf geom, expect, flag;      /* the device update stage's inputs */
     uint32_t *flag_host = nullptr;  /* pinned copy of flag */
     uint64_t expect_build = 0;      /* the build "expect" holds the flags of */
@@ -362,7 +362,15 @@ struct DevTables
             }
             if ((e = stage.end(st)) != hipSuccess) return e;
         }
+        if ((e = hot.reserve(sizeof(qr_dev_surf) * (size_t)h.n_surf)) != hipSuccess) return e;
+        if (send[2] && (e = qr_dev_surfaces((const qr_surface *)srf.ptr, h.n_surf,
+                                            (qr_dev_surf *)hot.ptr, st)) != hipSuccess)
+        {
+            sent[2].clear();
+            return e;
+        }
         t.surfaces = (qr_surface *)srf.ptr;
+        t.hot = (qr_dev_surf *)hot.ptr;
         t.materials = (qr_material *)mat.ptr;
         t.lights = (qr_light *)lgt.ptr;
         t.clips = (qr_clip *)clp.ptr;
@@ -383,7 +391,7 @@ struct DevTables
     }
     void release()
     {
-        srf.release(); mat.release(); lgt.release();
+        srf.release(); hot.release(); mat.release(); lgt.release();
         clp.release(); elem.release(); tex.release(); step.release();
         step_any.release(); refit_in.release(); refit_box.release();
         geom.release(); expect.release(); flag.release();
@@ -468,9 +476,9 @@ struct DevTables
         if ((e = stage.end(st)) != hipSuccess) return e;
         if (send_expect) expect_build = build_on_dev;
         e = qr_update_records((const qr_geom *)geom.ptr, h.n_surf, (const qr_clip *)clp.ptr,
-                              (qr_surface *)srf.ptr, (qr_material *)mat.ptr,
-                              (qr_refit_elem *)refit_in.ptr, (const int32_t *)expect.ptr,
-                              (uint32_t *)flag.ptr, st);
+                              (qr_surface *)srf.ptr, (qr_dev_surf *)hot.ptr,
+                              (qr_material *)mat.ptr, (qr_refit_elem *)refit_in.ptr,
+                              (const int32_t *)expect.ptr, (uint32_t *)flag.ptr, st);
         if (e != hipSuccess) return e;
         e = qr_refit_programs((qr_dev_step *)step.ptr, dev_n_step,
                               any ? (qr_dev_step *)step_any.ptr : nullptr, any ? dev_n_any : 0,

@@ -28,12 +28,16 @@
 #include "tracer_kernels.h"
 
 static __device__ __align__(256) uint8_t scratch[QRHIP_NOALLOC_BYTES];
+/* the walks' form of the surfaces, in an array of its own: as many records as
+ * the scratch array can hold surfaces, so it refuses no call */
+static __device__ __align__(256) qr_dev_surf scratch_hot[QRHIP_NOALLOC_BYTES / sizeof(qr_surface) + 1];
 
 namespace {
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
 uint8_t *g_scratch[MAX_DEVICES];   /* per device: the array's device address */
+qr_dev_surf *g_hot[MAX_DEVICES];   /* and scratch_hot's */
 
 /* the kernels' form of a culling program (DevTables::upload, dev_steps):
  * bounds grown by the box's share of the allowance; with src null, the
@@ -101,6 +105,11 @@ hipError_t noalloc_setup(int ordinal)
     e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return e;
     if (ptr == nullptr) return hipErrorInvalidSymbol;
+    void *hot = nullptr;
+    e = hipGetSymbolAddress(&hot, HIP_SYMBOL(scratch_hot));
+    if (e != hipSuccess) return e;
+    if (hot == nullptr) return hipErrorInvalidSymbol;
+    g_hot[ordinal] = (qr_dev_surf *)hot;
     g_scratch[ordinal] = (uint8_t *)ptr;
     return hipSuccess;
 }
@@ -198,9 +207,12 @@ int qrhip_render_tables_noalloc(qrhip_dev *dev, const qr_scene_tables *tab,
                            ref[0], ref[1], ref[2], dany);
     }
     HIP_TRY(hipGetLastError());
+    qr_dev_surf *hot = g_hot[dev->ordinal];
+    HIP_TRY(qr_dev_surfaces((const qr_surface *)(base + part[0].off), tab->n_surf, hot, st));
 
     qr_device_tables t;
     t.surfaces = (qr_surface *)(base + part[0].off);
+    t.hot = hot;
     t.materials = (qr_material *)(base + part[1].off);
     t.lights = (qr_light *)(base + part[2].off);
     t.clips = (qr_clip *)(base + part[3].off);

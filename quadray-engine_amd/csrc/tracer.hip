@@ -58,7 +58,7 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
         {
             if (primary) *hit_id = (sc.srf[h.srf].id << 1) | h.side;
             hit_info(sc, ray, h);
-            const V3 nrm = normal_at(sc, sc.srf[h.srf], h);
+            const V3 nrm = normal_at(sc, h);
             Node &nd = stk[sp];
             shade(sc, fd, ray, h, nrm, nd, [&](int, const Ray &sr) {
                 Hit sh;

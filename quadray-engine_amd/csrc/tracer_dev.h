@@ -50,19 +50,10 @@ __device__ __forceinline__ V3 pick(bool c, V3 a, V3 b)
 {
     return V3{c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z};
 }
-__device__ __forceinline__ float sel6(const V3 &a, const V3 &b, int i)
-{
-    return i < 3 ? sel(a, i) : sel(b, i - 3);
-}
 __device__ __forceinline__ void put(V3 &v, int i, float f)
 {
     if (i == 0) v.x = f; else if (i == 1) v.y = f; else v.z = f;
 }
-__device__ __forceinline__ void put6(V3 &a, V3 &b, int i, float f)
-{
-    if (i < 3) put(a, i, f); else put(b, i - 3, f);
-}
-
 /* x86 float->int conversion semantics: out of range and NaN give INT_MIN */
 __device__ __forceinline__ int32_t cvt_floor(float x)
 {
@@ -83,6 +74,7 @@ __device__ __forceinline__ int32_t cvt_rne(float x)
 struct Scene
 {
     const QC qr_surface  *srf;
+    const QC qr_dev_surf *hot;          /* the surfaces as the walks read them */
     const QC qr_material *mat;
     const QC qr_light    *lgt;
     const QC qr_clip     *clp;
@@ -99,6 +91,7 @@ inline Scene scene_of(const qr_device_tables *t)
 {
     Scene sc;
     sc.srf = (const QC qr_surface *)t->surfaces;
+    sc.hot = (const QC qr_dev_surf *)t->hot;
     sc.mat = (const QC qr_material *)t->materials;
     sc.lgt = (const QC qr_light *)t->lights;
     sc.clp = (const QC qr_clip *)t->clips;
@@ -132,64 +125,105 @@ struct Hit
     float u, v;
 };
 
-/* inverse-matrix product, diagonal first (tracer.cpp:2536-2568) */
-__device__ __forceinline__ V3 xform(const QC qr_surface &s, const V3 &d)
-{
-    V3 o;
-    o.x = s.tc[0][0] * d.x;
-    o.y = s.tc[1][1] * d.y;
-    o.z = s.tc[2][2] * d.z;
-    if (s.trm != 1)
-    {
-        o.x = o.x + s.tc[0][1] * d.y;
-        o.x = o.x + s.tc[0][2] * d.z;
-        o.y = o.y + s.tc[1][0] * d.x;
-        o.y = o.y + s.tc[1][2] * d.z;
-        o.z = o.z + s.tc[2][0] * d.x;
-        o.z = o.z + s.tc[2][1] * d.y;
-    }
-    return o;
-}
-
+/* inverse-matrix product, diagonal first (tracer.cpp:2536-2568); td its
+ * diagonal, to the rest */
 template <class P>
 __device__ __forceinline__ V3 sub3(const V3 &a, P p)
 {
     return V3{a.x - p[0], a.y - p[1], a.z - p[2]};
 }
 
-/* list-walk registers mirroring QuadRay's context fields */
-struct Walk
+__device__ __forceinline__ V3 xform_full(const float td[3], const float to[6], const V3 &d)
 {
-    V3  dff_x, dff_i;   /* DFF_X/Y/Z, DFF_I/J/K */
-    V3  ray_i;          /* RAY_I/J/K */
-    int cache_last;     /* trnode: last element of the group, -1 off */
-    int cache_first;    /* the group's transform-node element */
+    V3 o;
+    o.x = td[0] * d.x;
+    o.y = td[1] * d.y;
+    o.z = td[2] * d.z;
+    o.x = o.x + to[0] * d.y;
+    o.x = o.x + to[1] * d.z;
+    o.y = o.y + to[2] * d.x;
+    o.y = o.y + to[3] * d.z;
+    o.z = o.z + to[4] * d.x;
+    o.z = o.z + to[5] * d.y;
+    return o;
+}
+
+__device__ __forceinline__ V3 xform_diag(const float td[3], const V3 &d)
+{
+    return V3{td[0] * d.x, td[1] * d.y, td[2] * d.z};
+}
+
+/* the first 64 bytes of a qr_dev_surf, and the rest of its transform */
+struct SurfHead
+{
+    float    pos[3];
+    uint32_t flags;
+    float    sci[4];
+    float    scj[3];
+    float    d_eps, t_eps;
+    float    td[3];
+};
+static_assert(sizeof(SurfHead) == 64, "one scalar load");
+struct SurfOff
+{
+    float to[6];
+};
+struct SurfClip
+{
+    float cmin[3], cmax[3];
 };
 
-/* hit point and local hit of a root that passed clipping */
-struct ClipOut
+template <class T, class S>
+__device__ __forceinline__ T ldk(const QC S *p)
 {
-    V3 hit;             /* HIT */
-    V3 loc;             /* NEW: the local hit in the surface's tracing frame */
-};
+    T v;
+    __builtin_memcpy(&v, p, sizeof(T));
+    return v;
+}
+
+/* the record at byte offset "off" of the table (wave-uniform: one scalar
+ * load of 64 bytes) */
+__device__ __forceinline__ const QC qr_dev_surf *surf_at(const Scene &sc, uint32_t off)
+{
+    return (const QC qr_dev_surf *)((const QC char *)sc.hot + off);
+}
+
+__device__ __forceinline__ V3 xform(const SurfHead &s, const QC qr_dev_surf *p, const V3 &d)
+{
+    if ((s.flags & QR_DS_TRM) == QR_DS_TRM_DIAG) return xform_diag(s.td, d);
+    return xform_full(s.td, ldk<SurfOff>(p->to).to, d);
+}
+
+__device__ __forceinline__ int amap(uint32_t flags, int a)
+{
+    return (int)((flags >> (QR_DS_AMAP_BIT + 2 * a)) & 3u);
+}
+__device__ __forceinline__ int asgn(uint32_t flags, int a)
+{
+    return (int)((flags >> (QR_DS_ASGN_BIT + a)) & 1u);
+}
+/* scaler of world-aligned axis m */
+__device__ __forceinline__ float sci_at(const float sci[4], int m)
+{
+    return m == 0 ? sci[0] : (m == 1 ? sci[1] : sci[2]);
+}
 
 /* clipper evaluation (PL_clp 5696, QD_clp 6292, TP_clp 6466) */
-__device__ __forceinline__ bool clip_keep(const QC qr_surface &c, const V3 &nx,
-                                          const V3 &ni, int rel)
+__device__ __forceinline__ bool clip_keep(const SurfHead &c, const V3 &nx, const V3 &ni, int rel)
 {
+    const uint32_t kind = (c.flags >> QR_DS_CLP_BIT) & 3u;
+    const V3 p = pick((c.flags & QR_DS_SHIFT) != 0, ni, nx);
     float f;
-    if (c.clp_kind == 1)
+    if (kind == 1)
     {
-        int k = c.amap[2] + 3 * c.shift;
-        f = negif(sel6(nx, ni, k), c.asgn[2]);
+        f = negif(sel(p, amap(c.flags, 2)), asgn(c.flags, 2));
     }
     else
     {
-        const V3 p = pick(c.shift, ni, nx);
         float d0 = (p.x * p.x) * c.sci[0];
         float d1 = (p.y * p.y) * c.sci[1];
         float d2 = (p.z * p.z) * c.sci[2];
-        if (c.clp_kind == 2)
+        if (kind == 2)
         {
             d0 = d0 - (c.scj[0] + c.scj[0]) * p.x;
             d1 = d1 - (c.scj[1] + c.scj[1]) * p.y;
@@ -202,8 +236,74 @@ __device__ __forceinline__ bool clip_keep(const QC qr_surface &c, const V3 &nx,
     return rel < 0 ? (f >= 0.0f) : (f <= 0.0f);
 }
 
-/* depth test, local hit, apex snap, axis and custom clipping of one root
- * (CC_clp, tracer.cpp:2686-3236).
+/* wave masks: one bit per active lane where b holds, and back */
+__device__ __forceinline__ uint64_t lanes(bool b)
+{
+    return __builtin_amdgcn_ballot_w64(b);
+}
+__device__ __forceinline__ bool in_lane(uint64_t m)
+{
+    return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+
+/* apex snap of a local hit near a cone's or two planes' apex (tracer.cpp
+ * 2773-2944), for a root with a near-zero discriminant; dd: the ray's
+ * origin in the surface's tracing frame */
+__device__ __forceinline__ void apex_snap(uint32_t flags, const float sci[4], float t_eps,
+                                          const V3 &dd, int side, uint32_t amask, V3 &loc)
+{
+    const int ai = amap(flags, 0), aj = amap(flags, 1), ak = amap(flags, 2);
+    const bool two = (flags & QR_DS_APEX_TWO) != 0;
+    float li = sel(loc, ai);
+    float rr = li * li;
+    if (!two)
+    {
+        float lj = sel(loc, aj);
+        rr = rr + lj * lj;
+    }
+    float lk = sel(loc, ak);
+    rr = rr + lk * lk;
+    if (rr < t_eps)
+    {
+        float ci = bitsf((fbits(sel(dd, ai)) & SIGN) ^ fbits(1.0f));
+        float cj = 0.0f;
+        float sk = sci_at(sci, ai);
+        float lr = 1.0f;
+        if (!two)
+        {
+            cj = bitsf((fbits(sel(dd, aj)) & SIGN) ^ fbits(1.0f));
+            sk = sk + sci_at(sci, aj);
+            lr = lr + 1.0f;
+        }
+        sk = sk / sci_at(sci, ak);
+        sk = fxor(sk, SIGN);
+        float ck = sqrtf(sk);
+        float lc2 = sk + lr;
+        float inv = rsq(lc2);
+        inv = inv * t_eps;
+        ci = ci * inv;
+        cj = cj * inv;
+        ck = ck * inv;
+        uint32_t ts = side ? SIGN : 0u;
+        ck = fxor(ck, fbits(sel(dd, ak)) & SIGN);
+        ck = fxor(ck, (ts & amask) ^ amask);
+        uint32_t tsg = (ts | amask) ^ amask;
+        ci = fxor(ci, tsg);
+        cj = fxor(cj, tsg);
+        put(loc, ai, ci);
+        if (!two) put(loc, aj, cj);
+        put(loc, ak, ck);
+    }
+}
+
+__device__ __forceinline__ V3 ray_at(const V3 &dir, const V3 &org, float t)
+{
+    return V3{dir.x * t + org.x, dir.y * t + org.y, dir.z * t + org.z};
+}
+
+/* axis and custom clipping of one root at distance t (CC_clp, tracer.cpp
+ * 2686-3236) of the surface with record s at p, whose tracing frame has the
+ * ray rr from dd; the lanes that keep it.
  *
  * QuadRay keeps two local-hit registers, NEW_X (world-aligned, from HIT) and
  * NEW_I (transformed, from RAY_I and DFF_I): a surface with a transform
@@ -212,96 +312,52 @@ __device__ __forceinline__ bool clip_keep(const QC qr_surface &c, const V3 &nx,
  * NEW_X otherwise.  The engine only emits surfaces whose trm and shift
  * agree (a transformed surface always has a transform node, and a surface
  * under one always inherits its rotation), so the register read is always
- * the one refreshed for that root: one local hit, "loc". */
-__device__ bool clip_root(const Scene &sc, const Walk &w, const Ray &r, float t_buf,
-                          bool tie, const QC qr_surface &s, float t, int side,
-                          bool dmask, uint32_t amask, ClipOut *out = nullptr)
+ * the one refreshed for that root: one local hit. */
+__device__ __forceinline__ uint64_t clip_root(const Scene &sc, const Ray &r, const SurfHead &s,
+                                              uint32_t flags, const QC qr_dev_surf *p,
+                                              const V3 &rr, const V3 &dd, float t, uint64_t side,
+                                              uint64_t dmask, float a_val)
 {
-    /* the depth test is strict, but a nearest-hit walk takes a root equal to
-     * the kept one (tie): QuadRay walks camera rays and the secondary rays of
-     * reflecting and transparent surfaces over lists built in the reverse of
-     * the global list's order (core/engine/engine.cpp:2180-2420), so of two
-     * roots at the same distance the later one of the global list wins */
-    if (!(t_buf > t || (tie && t_buf == t)) || !(r.t_min < t)) return false;
-
-    V3 hit;
-    hit.x = r.dir.x * t + r.org.x;
-    hit.y = r.dir.y * t + r.org.y;
-    hit.z = r.dir.z * t + r.org.z;
-    const V3 ni = {w.ray_i.x * t + w.dff_i.x, w.ray_i.y * t + w.dff_i.y,
-                   w.ray_i.z * t + w.dff_i.z};
-    V3 loc = pick(s.shift != 0, ni, sub3(hit, s.pos));
-    const int sh = 3 * s.shift;
-
-    if (s.apex != 0 && dmask)
+    V3 hit = V3{0.0f, 0.0f, 0.0f};
+    if (!(flags & QR_DS_SHIFT) || (flags & QR_DS_CLIPS)) hit = ray_at(r.dir, r.org, t);
+    V3 loc;
+    if (flags & QR_DS_SHIFT) loc = ray_at(rr, dd, t);
+    else loc = sub3(hit, s.pos);
+    if ((flags & QR_DS_APEX) && dmask != 0)
     {
-        const int ai = s.amap[0], aj = s.amap[1], ak = s.amap[2];
-        const int mi = ai + sh, mj = aj + sh, mk = ak + sh;
-        float li = sel(loc, ai);
-        float rr = li * li;
-        if (s.apex != 2)
+        if (in_lane(dmask))
         {
-            float lj = sel(loc, aj);
-            rr = rr + lj * lj;
-        }
-        float lk = sel(loc, ak);
-        rr = rr + lk * lk;
-        if (rr < s.t_eps)
-        {
-            float ci = bitsf((fbits(sel6(w.dff_x, w.dff_i, mi)) & SIGN) ^ fbits(1.0f));
-            float cj = 0.0f;
-            float sk = s.sci[s.amap[0]];
-            float lr = 1.0f;
-            if (s.apex != 2)
-            {
-                cj = bitsf((fbits(sel6(w.dff_x, w.dff_i, mj)) & SIGN) ^ fbits(1.0f));
-                sk = sk + s.sci[s.amap[1]];
-                lr = lr + 1.0f;
-            }
-            sk = sk / s.sci[s.amap[2]];
-            sk = fxor(sk, SIGN);
-            float ck = sqrtf(sk);
-            float lc2 = sk + lr;
-            float inv = rsq(lc2);
-            inv = inv * s.t_eps;
-            ci = ci * inv;
-            cj = cj * inv;
-            ck = ck * inv;
-            uint32_t ts = side ? SIGN : 0u;
-            ck = fxor(ck, fbits(sel6(w.dff_x, w.dff_i, mk)) & SIGN);
-            ck = fxor(ck, (ts & amask) ^ amask);
-            uint32_t tsg = (ts | amask) ^ amask;
-            ci = fxor(ci, tsg);
-            cj = fxor(cj, tsg);
-            put(loc, ai, ci);
-            if (s.apex != 2) put(loc, aj, cj);
-            put(loc, ak, ck);
+            apex_snap(flags, s.sci, s.t_eps, dd, in_lane(side) ? 1 : 0, fbits(a_val) & SIGN, loc);
         }
     }
 
-    const V3 l = loc;
-    bool ok = true;
-    if ((s.cmin_on & 1) && !(s.cmin[0] <= l.x)) ok = false;
-    if ((s.cmin_on & 2) && !(s.cmin[1] <= l.y)) ok = false;
-    if ((s.cmin_on & 4) && !(s.cmin[2] <= l.z)) ok = false;
-    if ((s.cmax_on & 1) && !(s.cmax[0] >= l.x)) ok = false;
-    if ((s.cmax_on & 2) && !(s.cmax[1] >= l.y)) ok = false;
-    if ((s.cmax_on & 4) && !(s.cmax[2] >= l.z)) ok = false;
-
-    if (s.clip_cnt > 0)
+    uint64_t ok = ~0ull;
+    if (flags & QR_DS_AXIS_CLIP)
     {
-        bool saved = false;
+        const SurfClip c = ldk<SurfClip>(p->cmin);
+        if (flags & (1u << QR_DS_CMIN_BIT)) ok &= lanes(c.cmin[0] <= loc.x);
+        if (flags & (2u << QR_DS_CMIN_BIT)) ok &= lanes(c.cmin[1] <= loc.y);
+        if (flags & (4u << QR_DS_CMIN_BIT)) ok &= lanes(c.cmin[2] <= loc.z);
+        if (flags & (1u << QR_DS_CMAX_BIT)) ok &= lanes(c.cmax[0] >= loc.x);
+        if (flags & (2u << QR_DS_CMAX_BIT)) ok &= lanes(c.cmax[1] >= loc.y);
+        if (flags & (4u << QR_DS_CMAX_BIT)) ok &= lanes(c.cmax[2] >= loc.z);
+    }
+    if (flags & QR_DS_CLIPS)
+    {
+        const int beg = p->clip_beg, cnt = p->clip_cnt;
+        uint64_t saved = 0;
         int cache = -1;
         V3 nx = {0, 0, 0}, ni = {0, 0, 0};
-        for (int k = 0; k < s.clip_cnt; k++)
+        for (int k = 0; k < cnt; k++)
         {
-            const QC qr_clip &e = sc.clp[s.clip_beg + k];
-            if (e.kind == QR_CLIP_ENTER) { saved = ok; ok = true; continue; }
-            if (e.kind == QR_CLIP_LEAVE) { ok = !ok && saved; continue; }
-            const QC qr_surface &c = sc.srf[e.surf];
+            const qr_clip e = ldk<qr_clip>(&sc.clp[beg + k]);
+            if (e.kind == QR_CLIP_ENTER) { saved = ok; ok = ~0ull; continue; }
+            if (e.kind == QR_CLIP_LEAVE) { ok = ~ok & saved; continue; }
+            const QC qr_dev_surf *cp = &sc.hot[e.surf];
+            const SurfHead c = ldk<SurfHead>(cp);
             if (e.kind == QR_CLIP_TRNODE)
             {
-                if (e.surf == s.trnode)
+                if (e.surf == p->trnode)
                 {
                     nx.x = loc.x + s.pos[0];
                     nx.y = loc.y + s.pos[1];
@@ -309,7 +365,7 @@ __device__ bool clip_root(const Scene &sc, const Walk &w, const Ray &r, float t_
                 }
                 else
                 {
-                    nx = xform(c, sub3(hit, c.pos));
+                    nx = xform(c, cp, sub3(hit, c.pos));
                 }
                 cache = e.rel;
                 continue;
@@ -322,197 +378,168 @@ __device__ bool clip_root(const Scene &sc, const Walk &w, const Ray &r, float t_
             else
             {
                 nx = sub3(hit, c.pos);
-                if (c.trm != 0) ni = xform(c, nx);
+                if (c.flags & QR_DS_TRM) ni = xform(c, cp, nx);
             }
-            ok = ok && clip_keep(c, nx, ni, e.rel);
+            ok &= lanes(clip_keep(c, nx, ni, e.rel));
         }
-    }
-    if (out != nullptr)
-    {
-        out->hit = hit;
-        out->loc = loc;
     }
     return ok;
 }
 
-__device__ __forceinline__ bool shadows(uint32_t p)
-{
-    if (p & QR_PROP_LIGHT) return false;
-    if ((p & QR_PROP_TRANSP) && !(p & QR_PROP_REFRACT)) return false;
-    return true;
-}
-
-/* walk the surface list: nearest hit, or any shadowing hit (SHADOW) */
-/* transform set-up of list element e (surface record s; same: it is the
- * ray's origin surface) for ray r: the
- * DFF_X / DFF_I / RAY_I registers as QuadRay's list walk leaves them
- * (OO_loc, tracer.cpp:2466-2684); "last" opens a transform-node cache */
-__device__ __forceinline__ void elem_setup(Walk &w, const Ray &r,
-                                           const QC qr_surface &s, bool same,
-                                           int e, int last)
-{
-    if (same)
-    {
-        if (s.shift) w.dff_i = r.oloc; else w.dff_x = r.oloc;
-    }
-
-    if (s.tag >= 0 && w.cache_last >= 0)
-    {
-        if (!same) w.dff_i = sub3(w.dff_x, s.pos);
-        if (e == w.cache_last) w.cache_last = -1;
-    }
-    else
-    {
-        bool do_ray = same;
-        if (!same)
-        {
-            V3 d = sub3(r.org, s.pos);
-            w.dff_x = d;
-            if (s.trm != 0)
-            {
-                V3 t3 = xform(s, d);
-                if (s.tag < 0)
-                {
-                    w.dff_x = t3;
-                    w.cache_last = last;
-                    w.cache_first = e;
-                }
-                else
-                {
-                    w.dff_i = t3;
-                }
-                do_ray = true;
-            }
-        }
-        if (do_ray) w.ray_i = xform(s, r.dir);
-    }
-}
-
-/* roots of a quadric or two-plane surface in QuadRay's operation order */
+/* roots of a quadric or two-plane surface in the order they are tested:
+ * n1 / d1, then n2 / d2, undefined where the denominator is 0 */
 struct Roots
 {
-    float    t1, t2;
-    bool     t1m, t2m;      /* root defined (non-zero denominator) */
-    bool     dmask;         /* near-zero discriminant */
-    uint32_t amask;         /* sign of a */
-    int      first;         /* side tested first */
+    float n1, d1, n2, d2;
 };
 
-/* discriminant and roots (QD_rt1 5722-6206, TP_rt1 6337-6413); false when
- * the discriminant is negative */
-__device__ __forceinline__ bool solve(const QC qr_surface &s, const V3 &rr,
-                                      const V3 &dd, Roots &q)
+/* coefficients of the root equation (QD_rt1 5722-5900, TP_rt1 6337-6390) of
+ * the surface with flags, scalers sci and scj: rr, dd the ray's direction
+ * and origin in its tracing frame; returns the discriminant */
+__device__ __forceinline__ float quadric_abc(uint32_t flags, const float sci[4],
+                                             const float scj[3], const V3 &rr, const V3 &dd,
+                                             float &a_val, float &b_val, float &c_val)
 {
-    float a_val, b_val, c_val, d_val;
-    if (s.solver == QR_SOLVE_QUADRIC)
+    const uint32_t cls = flags & QR_DS_CLASS;
+    if (cls != QR_DC_TWOPLANE)
     {
-        float ax, bx, cx, ay, by, cy, az, bz, cz;
+        V3 sr, sd, sc;
+        if (cls == QR_DC_SPHERE)
         {
-            float sri = s.sci[0] * rr.x;
-            float sdi = s.sci[0] * dd.x;
-            sdi = sdi - s.scj[0];
-            ax = rr.x * sri;
-            bx = rr.x * sdi;
-            sdi = sdi - s.scj[0];
-            cx = dd.x * sdi;
+            sr = rr;
+            sd = sc = dd;
         }
+        else
         {
-            float sri = s.sci[1] * rr.y;
-            float sdi = s.sci[1] * dd.y;
-            sdi = sdi - s.scj[1];
-            ay = rr.y * sri;
-            by = rr.y * sdi;
-            sdi = sdi - s.scj[1];
-            cy = dd.y * sdi;
+            sr = V3{sci[0] * rr.x, sci[1] * rr.y, sci[2] * rr.z};
+            sd = sc = V3{sci[0] * dd.x, sci[1] * dd.y, sci[2] * dd.z};
+            if (cls == QR_DC_QUADRIC)
+            {
+                sd = sub3(sd, scj);
+                sc = sub3(sd, scj);
+            }
         }
-        {
-            float sri = s.sci[2] * rr.z;
-            float sdi = s.sci[2] * dd.z;
-            sdi = sdi - s.scj[2];
-            az = rr.z * sri;
-            bz = rr.z * sdi;
-            sdi = sdi - s.scj[2];
-            cz = dd.z * sdi;
-        }
-        a_val = ax + ay;
-        b_val = bx + by;
-        c_val = cx + cy;
-        a_val = a_val + az;
-        b_val = b_val + bz;
-        c_val = c_val + cz;
-        c_val = c_val - s.sci[3];
-        d_val = b_val * b_val - c_val * a_val;
+        a_val = rr.x * sr.x + rr.y * sr.y;
+        b_val = rr.x * sd.x + rr.y * sd.y;
+        c_val = dd.x * sc.x + dd.y * sc.y;
+        a_val = a_val + rr.z * sr.z;
+        b_val = b_val + rr.z * sd.z;
+        c_val = c_val + dd.z * sc.z;
+        c_val = c_val - sci[3];
+        return b_val * b_val - c_val * a_val;
     }
-    else
-    {
-        const int mi = s.amap[0], mk = s.amap[2];
-        float ri = sel(rr, mi), di = sel(dd, mi);
-        float rk = sel(rr, mk), dk = sel(dd, mk);
-        float si_ = s.sci[mi], sk_ = s.sci[mk];
-        float dx = di * rk - dk * ri;
-        dx = dx * dx;
-        dx = dx * si_;
-        dx = dx * sk_;
-        d_val = fabsf(dx);
-        float bi = si_ * di, bk = sk_ * dk;
-        bi = bi * ri;
-        bk = bk * rk;
-        b_val = bi + bk;
-        float ci = di * di, ck = dk * dk;
-        ci = ci * si_;
-        ck = ck * sk_;
-        c_val = ci + ck;
-        float ai = ri * ri, ak = rk * rk;
-        ai = ai * si_;
-        ak = ak * sk_;
-        a_val = ai + ak;
-    }
+    const int mi = amap(flags, 0), mk = amap(flags, 2);
+    float ri = sel(rr, mi), di = sel(dd, mi);
+    float rk = sel(rr, mk), dk = sel(dd, mk);
+    float si_ = sci_at(sci, mi), sk_ = sci_at(sci, mk);
+    float dx = di * rk - dk * ri;
+    dx = dx * dx;
+    dx = dx * si_;
+    dx = dx * sk_;
+    float bi = si_ * di, bk = sk_ * dk;
+    bi = bi * ri;
+    bk = bk * rk;
+    b_val = bi + bk;
+    float ci = di * di, ck = dk * dk;
+    ci = ci * si_;
+    ck = ck * sk_;
+    c_val = ci + ck;
+    float ai = ri * ri, ak = rk * rk;
+    ai = ai * si_;
+    ak = ak * sk_;
+    a_val = ai + ak;
+    return fabsf(dx);
+}
 
-    if (!(0.0f <= d_val)) return false;
+/* the correctly rounded square root of x in [2^-96, inf] (sqrtf's own steps
+ * without those for smaller values): the hardware root, corrected by the
+ * signs of the residuals of its neighbours */
+__device__ __forceinline__ float sqrt_mid(float x)
+{
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float lo = bitsf(fbits(s) - 1u), hi = bitsf(fbits(s) + 1u);
+    float q = __builtin_fmaf(-lo, s, x) <= 0.0f ? lo : s;
+    q = __builtin_fmaf(-hi, s, x) > 0.0f ? hi : q;
+    return q;
+}
+constexpr float SQRT_MID_MIN = 1.2621774483536189e-29f;     /* 2^-96 */
+
+/* roots from the coefficients and a discriminant >= 0, any of them
+ * (QD_rt1 5900-6206, TP_rt1 6390-6413); side 1 (root 2) is tested first
+ * where a < 0.  A near-zero discriminant's roots are formed here, as a
+ * quotient by 1 (exact) or, where undefined, by 0. */
+__device__ void roots_any(float a_val, float b_val, float c_val, float d_val, float d_eps,
+                          float t_eps, Roots &q)
+{
     float nb = -b_val;
-    q.dmask = d_val < s.d_eps;
     float sd = sqrtf(d_val);
     sd = fxor(sd, fbits(nb) & SIGN);
     float qq = nb + sd;
     const bool m_pos = 0.0f <= sd;
     const bool m_neg = 0.0f > sd;
-    float t1n = m_neg ? qq : (m_pos ? c_val : 0.0f);
-    float t1d = m_neg ? a_val : (m_pos ? qq : 0.0f);
-    float t2n = m_neg ? c_val : (m_pos ? qq : 0.0f);
-    float t2d = m_neg ? qq : (m_pos ? a_val : 0.0f);
-    q.amask = fbits(a_val) & SIGN;
-
-    if (q.dmask)
+    float n1 = m_neg ? qq : (m_pos ? c_val : 0.0f);
+    float d1 = m_neg ? a_val : (m_pos ? qq : 0.0f);
+    float n2 = m_neg ? c_val : (m_pos ? qq : 0.0f);
+    float d2 = m_neg ? qq : (m_pos ? a_val : 0.0f);
+    const uint32_t amask = fbits(a_val) & SIGN;
+    if (d_val < d_eps)
     {
-        if (t1n == 0.0f) t1d = 1.0f;
-        if (t2n == 0.0f) t2d = 1.0f;
-        float t1 = t1n / t1d;
-        float t2 = t2n / t2d;
-        q.t1m = t1d != 0.0f;
-        q.t2m = t2d != 0.0f;
+        if (n1 == 0.0f) d1 = 1.0f;
+        if (n2 == 0.0f) d2 = 1.0f;
+        float t1 = n1 / d1;
+        float t2 = n2 / d2;
+        const bool t1m = d1 != 0.0f, t2m = d2 != 0.0f;
         float tdf = t1 - t2;
-        tdf = fxor(tdf, q.amask);
+        tdf = fxor(tdf, amask);
         bool fm = 0.0f <= tdf;
         if (!fm) tdf = 0.0f;
-        float te = fm ? s.t_eps : 0.0f;
+        float te = fm ? t_eps : 0.0f;
         te = te * t1;
         te = fabsf(te);
         tdf = tdf * -0.5f;
         tdf = tdf - te;
-        tdf = fxor(tdf, q.amask);
-        if (!(q.t1m && q.t2m)) tdf = 0.0f;
-        q.t1 = t1 + tdf;
-        q.t2 = t2 - tdf;
+        tdf = fxor(tdf, amask);
+        if (!(t1m && t2m)) tdf = 0.0f;
+        n1 = t1 + tdf;
+        n2 = t2 - tdf;
+        d1 = t1m ? 1.0f : 0.0f;
+        d2 = t2m ? 1.0f : 0.0f;
     }
-    else
-    {
-        q.t1 = t1n / t1d;
-        q.t2 = t2n / t2d;
-        q.t1m = t1d != 0.0f;
-        q.t2m = t2d != 0.0f;
-    }
-    q.first = (0.0f > a_val) ? 1 : 0;
-    return true;
+    const bool second = 0.0f > a_val;
+    q.n1 = second ? n2 : n1;
+    q.d1 = second ? d2 : d1;
+    q.n2 = second ? n1 : n2;
+    q.d2 = second ? d1 : d2;
+}
+
+/* the same for a discriminant >= d_eps and in sqrt_mid's range: the signed
+ * root of it is not 0, so root 1 is qq / a and root 2 c / qq where b > 0
+ * (or +0), the other way round elsewhere */
+__device__ __forceinline__ void roots_mid(float a_val, float b_val, float c_val, float d_val,
+                                          uint64_t second, Roots &q)
+{
+    const float nb = -b_val;
+    const float qq = nb + __builtin_copysignf(sqrt_mid(d_val), nb);
+    const bool x = in_lane(lanes((int32_t)fbits(nb) < 0) ^ second);
+    q.n1 = x ? qq : c_val;
+    q.d1 = x ? a_val : qq;
+    q.n2 = x ? c_val : qq;
+    q.d2 = x ? qq : a_val;
+}
+
+/* the lanes whose n / d, rounded, may lie above t_min and at or below
+ * t_lim, given the next float above t_lim; never without one that does.  With n'
+ * = n times the sign of d and d' = |d|: rounding is monotonic and t_min a
+ * float, so round(n/d) > t_min means n'/d' > t_min, n' > t_min * d' and, n'
+ * being a float, n' >= round(t_min * d'); likewise above.  A zero or NaN
+ * denominator's root is undefined, or rejected by the exact comparisons
+ * that follow. */
+template <bool T0>
+__device__ __forceinline__ uint64_t roots_near(float n, float d, float t_min, float t_next)
+{
+    const float nn = fxor(n, fbits(d) & SIGN);
+    const float lo = T0 ? 0.0f : t_min * fabsf(d);
+    return lanes(nn >= lo) & lanes(nn <= t_next * fabsf(d));
 }
 
 /* reciprocal of a direction component for the slab tests: approximate, and
@@ -586,85 +613,13 @@ __device__ __forceinline__ bool box_pass(const qr_dev_step &st, const BoxRay &b,
     return fmaxf(tn, t_min) <= fminf(tf, t_buf);
 }
 
-/* material properties of one side of a surface at a per-lane side: both
- * read as wave-uniform scalars, then selected (an indexed read would be a
- * vector memory load) */
-__device__ __forceinline__ uint32_t side_props(const QC qr_surface &s, int side)
-{
-    const uint32_t p0 = __builtin_amdgcn_readfirstlane(s.props[0]);
-    const uint32_t p1 = __builtin_amdgcn_readfirstlane(s.props[1]);
-    return side ? p1 : p0;
-}
-
-/* one root of a quadric (side 0: t1, side 1: t2) through the origin-side
- * rule, the depth test and clipping; true when it is accepted */
-__device__ __forceinline__ bool try_root(const Scene &sc, Walk &w, const Ray &r,
-                                         float t_buf, bool tie, const QC qr_surface &s,
-                                         const Roots &q, int side, bool same)
-{
-    const int fl = r.flags & 3;
-    if (same && (fl == 1 - side || fl == 2 + side)) return false;
-    const float t = side == 0 ? q.t1 : q.t2;
-    const bool tm = side == 0 ? q.t1m : q.t2m;
-    if (!tm) return false;
-    return clip_root(sc, w, r, t_buf, tie, s, t, side, q.dmask, q.amask);
-}
-
 /* whether QuadRay gives a surface a nearest-hit list of its own for the
  * rays leaving it (reflecting or not opaque on either side,
  * core/engine/engine.cpp:2180-2201), built in the reverse of the global
  * list's order; other surfaces' rays walk the global list itself */
-__device__ __forceinline__ bool own_list(const QC qr_surface &s)
+__device__ __forceinline__ bool own_list(const Scene &sc, int surf)
 {
-    const uint32_t p0 = s.props[0], p1 = s.props[1];
-    return ((p0 | p1) & QR_PROP_REFLECT) != 0 || (p0 & p1 & QR_PROP_OPAQUE) == 0;
-}
-
-/* the roots of list element e (surface s, set up in w) for ray r that the
- * walk accepts: true with the accepted side and distance.  A tie goes by
- * list order ("rev": the later element wins), or with SPATIAL by element
- * index against best_e. */
-template <bool SHADOW, bool SPATIAL>
-__device__ __forceinline__ bool elem_roots(const Scene &sc, Walk &w, const Ray &r,
-                                           const QC qr_surface &s, bool same, int e,
-                                           const Hit &best, int best_e, bool rev, float t_buf,
-                                           int &side, float &t)
-{
-    const int sh = 3 * s.shift;
-    bool acc = false;
-    if (s.solver == QR_SOLVE_PLANE)
-    {
-        const int k = s.amap[2] + sh;
-        float dff_k = negif(sel6(w.dff_x, w.dff_i, k), s.asgn[2]);
-        float ray_k = negif(k < 3 ? sel(r.dir, k) : sel(w.ray_i, k - 3), s.asgn[2]);
-        dff_k = -dff_k;
-        if (!same && ray_k != 0.0f)
-        {
-            t = dff_k / ray_k;
-            side = ray_k < 0.0f ? 0 : 1;
-            const bool tie = !SHADOW && best.srf >= 0 &&
-                             (SPATIAL ? (rev ? e > best_e : e < best_e) : rev);
-            acc = clip_root(sc, w, r, t_buf, tie, s, t, side, false, 0u);
-        }
-    }
-    else
-    {
-        Roots q;
-        if (solve(s, pick(s.shift, w.ray_i, r.dir), pick(s.shift, w.dff_i, w.dff_x), q))
-        {
-            const bool tie = !SHADOW && best.srf >= 0 &&
-                             (SPATIAL ? (rev ? e > best_e : e < best_e) : rev);
-            side = q.first;
-            acc = try_root(sc, w, r, t_buf, tie, s, q, side, same);
-            if (!acc)
-            {
-                side = 1 - side;
-                acc = try_root(sc, w, r, t_buf, tie, s, q, side, same);
-            }
-            t = side == 0 ? q.t1 : q.t2;
-        }
-    }
-    return acc;
+    return (sc.hot[surf].flags & QR_DS_OWN_LIST) != 0;
 }
 
 /* most work-items in a workgroup of a kernel that walks the surface list */
@@ -677,36 +632,56 @@ __device__ __forceinline__ bool elem_roots(const Scene &sc, Walk &w, const Ray &
  * order wins, or with "rev" the last: camera rays, and the rays leaving a
  * surface that has its own list (own_list: every secondary ray of the
  * Whitted tracer), walk lists that QuadRay builds in the reverse of this
- * one's order.
+ * one's order.  T0: the ray's t_min is 0.
  *
  * The loop has one exit, taken by the whole wave: a lane whose shadow test
  * is decided stops keeping boxes open, and the wave leaves once every lane
  * is decided (a lane leaving on its own would split the loop's exit and cost
- * every iteration a per-lane state dispatch). */
-template <bool SHADOW, bool SPATIAL = false>
+ * every iteration a per-lane state dispatch).
+ *
+ * An element's registers (DFF_X / DFF_I / RAY_I of QuadRay's list walk,
+ * OO_loc, tracer.cpp:2466-2684) are the ray's origin and direction in the
+ * frame of the surface (dd, rr) and of the open transform node (node_o,
+ * node_d).  What decides between them is the same for the whole wave, so
+ * the branches are scalar; only a ray leaving the surface itself differs,
+ * which takes its origin's local hit.  Which lanes keep a root is held in
+ * wave masks: no branch of the element work changes the active lanes, but
+ * for the rare near-zero discriminants and apexes.
+ *
+ * What bounds it is VALU issue (the path tracer's bounces issue a VALU
+ * instruction in 92% of their quad cycles), so a quadric takes only what its
+ * class needs, its quotients are formed only for roots that can lie in the
+ * ray's range, and a hit point only where the surface clips.  Against one
+ * division per root and one clipping stage per root for every surface, read
+ * from the 208-byte record: the bounces of a 1280x720 64-spp frame issue
+ * 1.77e10 wave-level VALU instructions instead of 2.09e10, and 6.5e8 scalar
+ * loads instead of 2.2e9 (the frame 37.5 -> 31.4 ms); a 641x359 4X frame of
+ * glass 2.51 -> 2.21 ms, a 1080p 4X frame of 64 quadrics 2.11 -> 2.06 ms with
+ * its copy to the host.  One body for both roots also makes the walks' code
+ * a third shorter. */
+template <bool SHADOW, bool T0 = SHADOW>
 __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
 {
-    Walk w;
-    w.cache_last = -1;
-    w.cache_first = 0;
-    w.dff_x = V3{0, 0, 0};
-    w.dff_i = V3{0, 0, 0};
-    w.ray_i = V3{0, 0, 0};
-    float t_buf = r.t_max;
-    best.srf = -1;
-    bool shadowed = false;
+    V3 node_o = V3{0, 0, 0};
+    V3 node_d = V3{0, 0, 0};
+    int cache_last = -1;    /* trnode: last element of the group, -1 off */
+    int cache_first = 0;    /* the group's transform-node element */
+    /* The largest distance wanted.  The depth test is strict, but a
+     * nearest-hit walk takes a root equal to the kept one (a tie, "rev"), so
+     * the limit is the kept distance itself or the float below it; with no
+     * hit yet no root ties with t_max. */
+    const uint32_t below = rev ? 0u : 1u;
+    float t_lim = bitsf(fbits(r.t_max) - 1u);
+    int kept = -1;          /* record's byte offset | side */
     /* lanes that still keep boxes open (any-hit walks: not yet shadowed),
      * as a wave mask that the box tests' ballots are masked with */
-    uint64_t live = ~0ull;
+    uint64_t live = lanes(true);
 
     /* the ray's side of the world boxes (the reciprocal direction is
      * approximate: the boxes carry an allowance far above its error) */
     const BoxRay br = box_ray(r.org, r.dir, sc.ref_x, sc.ref_y, sc.ref_z);
 
-    /* nearest-hit walks over the spatial (any-hit) program visit units out
-     * of list order: exact ties then go by element index (best_e) */
-    const QC qr_dev_step *prog = SHADOW || SPATIAL ? sc.step_any : sc.step;
-    int best_e = -1;
+    const QC qr_dev_step *prog = SHADOW ? sc.step_any : sc.step;
     /* the ray's side of the open transform-node group's member boxes, in the
      * node's frame: kept in LDS, a slot per work-item, not in registers the
      * whole loop would hold.  A member's step is reached only through its
@@ -716,7 +691,7 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
     const unsigned tid = threadIdx.x;
     /* the byte offset of the ray's origin surface record (none: matches no
      * record) */
-    const uint32_t org_off = r.origin >= 0 ? (uint32_t)r.origin * (uint32_t)sizeof(qr_surface)
+    const uint32_t org_off = r.origin >= 0 ? (uint32_t)r.origin * (uint32_t)sizeof(qr_dev_surf)
                                            : 0xffffffffu;
     /* two loops: the inner one runs the box steps up to the next element
      * step and touches no walk register, so the element work is the only
@@ -731,7 +706,7 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
         qr_dev_step st = step_at(prog, off);
         while (st.elem < 0)
         {
-            const uint64_t near = __builtin_amdgcn_ballot_w64(box_pass(st, br, r.t_min, t_buf));
+            const uint64_t near = lanes(box_pass(st, br, r.t_min, t_lim));
             off = (near & live) != 0 ? off + QR_DEV_STEP_BYTES : (uint32_t)st.skip;
             st = step_at(prog, off);
         }
@@ -756,118 +731,289 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
             gb.hx = s_gb[6][tid];
             gb.hy = s_gb[7][tid];
             gb.hz = s_gb[8][tid];
-            keep &= __builtin_amdgcn_ballot_w64(box_pass(st, gb, r.t_min, t_buf));
+            keep &= lanes(box_pass(st, gb, r.t_min, t_lim));
         }
         if (keep != 0)
         {
+            /* the record's byte offset (the index only for a kept hit), and
+             * its head: one load */
+            const uint32_t soff = (uint32_t)st.skip & ~3u;
+            const QC qr_dev_surf *const sp = surf_at(sc, soff);
+            const SurfHead s = ldk<SurfHead>(sp);
             /* the cache holds only inside its group, whose last element may
              * have been skipped (the any-hit program also visits groups out
              * of list order) */
-            if (w.cache_last >= 0 && (e > w.cache_last || e < w.cache_first))
+            if (e > cache_last || e < cache_first) cache_last = -1;
+            V3 rr, dd;
+            if (cache_last >= 0 && (s.flags & QR_DS_NODE) == 0)
             {
-                w.cache_last = -1;
+                dd = sub3(node_o, s.pos);
+                rr = node_d;
+                if (e == cache_last) cache_last = -1;
             }
-            /* the record's byte offset (the index only for a kept hit) */
-            const uint32_t soff = (uint32_t)st.skip & ~3u;
-            const QC qr_surface &s = *(const QC qr_surface *)((const QC char *)sc.srf + soff);
-            const bool same = soff == org_off;
-            /* a transform node's group end (only a node's step has one;
-             * other surfaces ignore it) */
-            const int last = __float_as_int(st.lo[0]);
-            elem_setup(w, r, s, same, e, last);
-            if (s.tag < 0 && s.trm != 0)
+            else
             {
-                /* a transform node (never a ray's origin) opened its group:
-                 * the ray in the node's frame, about the node's origin */
-                const BoxRay gb = box_ray(w.dff_x, w.ray_i, 0.0f, 0.0f, 0.0f);
-                s_gb[0][tid] = gb.ix;
-                s_gb[1][tid] = gb.iy;
-                s_gb[2][tid] = gb.iz;
-                s_gb[3][tid] = gb.lx;
-                s_gb[4][tid] = gb.ly;
-                s_gb[5][tid] = gb.lz;
-                s_gb[6][tid] = gb.hx;
-                s_gb[7][tid] = gb.hy;
-                s_gb[8][tid] = gb.hz;
+                dd = sub3(r.org, s.pos);
+                rr = r.dir;
+                if (s.flags & QR_DS_TRM)
+                {
+                    if ((s.flags & QR_DS_TRM) != QR_DS_TRM_DIAG)
+                    {
+                        const SurfOff o = ldk<SurfOff>(sp->to);
+                        dd = xform_full(s.td, o.to, dd);
+                        rr = xform_full(s.td, o.to, rr);
+                    }
+                    else
+                    {
+                        dd = xform_diag(s.td, dd);
+                        rr = xform_diag(s.td, rr);
+                    }
+                    if (s.flags & QR_DS_NODE)
+                    {
+                        /* a transform node (never a ray's origin) opens its
+                         * group, whose end its step holds: the ray in the
+                         * node's frame, about the node's origin */
+                        node_o = dd;
+                        node_d = rr;
+                        cache_last = __float_as_int(st.lo[0]);
+                        cache_first = e;
+                        const BoxRay gb = box_ray(dd, rr, 0.0f, 0.0f, 0.0f);
+                        s_gb[0][tid] = gb.ix;
+                        s_gb[1][tid] = gb.iy;
+                        s_gb[2][tid] = gb.iz;
+                        s_gb[3][tid] = gb.lx;
+                        s_gb[4][tid] = gb.ly;
+                        s_gb[5][tid] = gb.lz;
+                        s_gb[6][tid] = gb.hx;
+                        s_gb[7][tid] = gb.hy;
+                        s_gb[8][tid] = gb.hz;
+                    }
+                }
             }
-            if (s.solver != QR_SOLVE_NONE)
+            const uint64_t same = lanes(soff == org_off);
+            if (same != 0)
+            {
+                const bool m = in_lane(same);
+                dd = pick(m, r.oloc, dd);
+            }
+            const uint32_t cls = s.flags & QR_DS_CLASS;
+            if (cls != QR_SOLVE_NONE)
             {
                 if (kind == QR_LOCAL_OWN)
                 {
                     /* the surface's own box, in its tracing frame (the
                      * registers the roots are computed from), whose
                      * reference point is the surface's origin */
-                    const BoxRay bl = box_ray(w.dff_i, w.ray_i, 0.0f, 0.0f, 0.0f);
-                    keep &= __builtin_amdgcn_ballot_w64(box_pass(st, bl, r.t_min, t_buf));
+                    const BoxRay bl = box_ray(dd, rr, 0.0f, 0.0f, 0.0f);
+                    keep &= lanes(box_pass(st, bl, r.t_min, t_lim));
                 }
                 if (keep != 0)
                 {
-                    int side = 0;
-                    float t = 0.0f;
-                    const bool acc = elem_roots<SHADOW, SPATIAL>(sc, w, r, s, same, e, best,
-                                                                 best_e, rev, t_buf, side, t);
-                    if (SHADOW)
+                    const float t_next = bitsf(fbits(t_lim) + 1u);
+                    /* the lanes with a first and a second root, and those
+                     * whose first is of side 1 */
+                    uint64_t m1, m2 = 0, side, dmask = 0;
+                    float n, d, a_val = 0.0f, n2 = 0.0f, d2 = 0.0f;
+                    if (cls == QR_DC_PLANE)
                     {
-                        shadowed = shadowed || (acc && shadows(side_props(s, side)));
-                        live = __builtin_amdgcn_ballot_w64(!shadowed);
-                        if (live == 0) break;
+                        const int k = amap(s.flags, 2);
+                        if (k == 0)
+                        {
+                            n = -dd.x;
+                            d = rr.x;
+                        }
+                        else if (k == 1)
+                        {
+                            n = -dd.y;
+                            d = rr.y;
+                        }
+                        else
+                        {
+                            n = -dd.z;
+                            d = rr.z;
+                        }
+                        /* (-dff) / ray, both negated where the plane's axis
+                         * is: the quotient is the same */
+                        side = lanes(!(d < 0.0f));
+                        if (asgn(s.flags, 2)) side = lanes(!(d > 0.0f));
+                        m1 = roots_near<T0>(n, d, r.t_min, t_next) & ~same;
                     }
-                    else if (acc)
+                    else
                     {
-                        t_buf = t;
-                        best_e = e;
-                        best.srf = (int)(soff / (uint32_t)sizeof(qr_surface));
-                        best.side = side;
-                        best.t = t;
+                        float b_val, c_val;
+                        const float d_val = quadric_abc(s.flags, s.sci, s.scj, rr, dd, a_val,
+                                                        b_val, c_val);
+                        m1 = lanes(0.0f <= d_val);
+                        side = 0;
+                        n = d = 0.0f;
+                        if (m1 != 0)
+                        {
+                            side = lanes(0.0f > a_val);
+                            Roots q;
+                            dmask = lanes(d_val < s.d_eps) & m1;
+                            if (dmask != 0 || !(s.d_eps >= SQRT_MID_MIN))
+                            {
+                                roots_any(a_val, b_val, c_val, d_val, s.d_eps, s.t_eps, q);
+                            }
+                            else
+                            {
+                                roots_mid(a_val, b_val, c_val, d_val, side, q);
+                            }
+                            n = q.n1;
+                            d = q.d1;
+                            n2 = q.n2;
+                            d2 = q.d2;
+                            m2 = roots_near<T0>(n2, d2, r.t_min, t_next) & m1;
+                            m1 &= roots_near<T0>(n, d, r.t_min, t_next);
+                            if (same != 0)
+                            {
+                                /* a ray leaving this surface skips the root
+                                 * it starts from: the other side's, or its
+                                 * own when it passes through */
+                                const uint64_t own = lanes((r.flags & 1) != 0) ^
+                                                     lanes((r.flags & 2) == 0);
+                                m1 &= ~(same & ~(own ^ side));
+                                m2 &= ~(same & (own ^ side));
+                            }
+                        }
                     }
+                    /* the roots in their order: the second only where the
+                     * first is not accepted */
+                    uint64_t take = m1 | m2;
+                    while (take != 0)
+                    {
+                        /* (the flags' tests stay inside the loop: hoisted,
+                         * their lane masks do not fit the scalar registers) */
+                        uint32_t flags = s.flags;
+                        asm volatile("" : "+s"(flags));
+                        const uint64_t use2 = take & ~m1;
+                        if (use2 != 0)
+                        {
+                            const bool u = in_lane(use2);
+                            n = u ? n2 : n;
+                            d = u ? d2 : d;
+                            side ^= use2;
+                        }
+                        const float t = n / d;
+                        uint64_t acc = take & lanes(t <= t_lim) & lanes(r.t_min < t);
+                        if ((flags & (QR_DS_AXIS_CLIP | QR_DS_CLIPS)) && acc != 0)
+                        {
+                            acc &= clip_root(sc, r, s, flags, sp, rr, dd, t, side, dmask, a_val);
+                        }
+                        take = m1 & m2 & ~acc;
+                        m1 = 0;
+                        if (SHADOW)
+                        {
+                            uint64_t cast = 0;
+                            if (flags & (1u << QR_DS_SHADOW_BIT)) cast |= ~side;
+                            if (flags & (2u << QR_DS_SHADOW_BIT)) cast |= side;
+                            live &= ~(acc & cast);
+                        }
+                        else
+                        {
+                            const bool u = in_lane(acc);
+                            t_lim = u ? bitsf(fbits(t) - below) : t_lim;
+                            const int code = (int)soff | (in_lane(side) ? 1 : 0);
+                            kept = u ? code : kept;
+                        }
+                    }
+                    if (SHADOW && live == 0) break;
                 }
             }
         }
     }
-    return SHADOW ? shadowed : best.srf >= 0;
+    if (SHADOW) return !in_lane(live);
+    best.srf = kept < 0 ? -1 : kept / (int)sizeof(qr_dev_surf);
+    best.side = kept & 1;
+    best.t = bitsf(fbits(t_lim) + below);
+    return kept >= 0;
 }
 
 /* hit point, local hit and plane texture coordinates of an accepted root,
  * recomputed with the operations the walk applied to it: the element set-up
- * (after its transform node's, for a grouped surface), the roots and the
- * clipping stage of that surface */
+ * (after its transform node's, for a grouped surface), the roots' apex snap
+ * and the local hit of that surface */
 __device__ void hit_info(const Scene &sc, const Ray &r, Hit &h)
 {
-    Walk w;
-    w.cache_last = -1;
-    w.cache_first = 0;
-    w.dff_x = V3{0, 0, 0};
-    w.dff_i = V3{0, 0, 0};
-    w.ray_i = V3{0, 0, 0};
-    const QC qr_surface &s = sc.srf[h.srf];
-    if (s.tag >= 0 && s.trnode >= 0 && s.trnode != h.srf)
+    const QC qr_dev_surf &s = sc.hot[h.srf];
+    const uint32_t flags = s.flags;
+    const bool same = h.srf == r.origin;
+    const float td[3] = {s.td[0], s.td[1], s.td[2]};
+    const V3 pos = V3{s.pos[0], s.pos[1], s.pos[2]};
+    V3 dd, rr;
+    bool cached = false;
+    const int node = s.trnode;
+    if ((flags & QR_DS_NODE) == 0 && node >= 0 && node != h.srf)
     {
-        const QC qr_surface &tn = sc.srf[s.trnode];
-        if (tn.tag < 0 && tn.trm != 0)
+        const QC qr_dev_surf &n = sc.hot[node];
+        const uint32_t nf = n.flags;
+        if ((nf & QR_DS_NODE) != 0 && (nf & QR_DS_TRM) != 0)
         {
-            elem_setup(w, r, tn, s.trnode == r.origin, -2, 0x7fffffff);
+            const float nd[3] = {n.td[0], n.td[1], n.td[2]};
+            const V3 d = sub3(r.org, n.pos);
+            if ((nf & QR_DS_TRM) != QR_DS_TRM_DIAG)
+            {
+                const float to[6] = {n.to[0], n.to[1], n.to[2], n.to[3], n.to[4], n.to[5]};
+                dd = xform_full(nd, to, d);
+                rr = xform_full(nd, to, r.dir);
+            }
+            else
+            {
+                dd = xform_diag(nd, d);
+                rr = xform_diag(nd, r.dir);
+            }
+            cached = true;
         }
     }
-    elem_setup(w, r, s, h.srf == r.origin, -1, -1);
-    bool dmask = false;
-    uint32_t amask = 0u;
-    if (s.solver != QR_SOLVE_PLANE)
+    if (cached)
     {
-        Roots q;
-        solve(s, pick(s.shift, w.ray_i, r.dir), pick(s.shift, w.dff_i, w.dff_x), q);
-        dmask = q.dmask;
-        amask = q.amask;
+        if (flags & QR_DS_SHIFT)
+        {
+            dd = V3{dd.x - pos.x, dd.y - pos.y, dd.z - pos.z};
+        }
+        else
+        {
+            rr = r.dir;     /* dff_x: the node's */
+        }
     }
-    ClipOut co;
-    co.hit = V3{0, 0, 0};
-    co.loc = V3{0, 0, 0};
-    clip_root(sc, w, r, 3.402823466e+38f, false, s, h.t, h.side, dmask, amask, &co);
-    h.hit = co.hit;
-    h.loc = co.loc;
-    if (s.solver == QR_SOLVE_PLANE)
+    else
     {
-        h.u = negif(sel(co.loc, s.amap[0]), s.asgn[0]);
-        h.v = negif(sel(co.loc, s.amap[1]), s.asgn[1]);
+        dd = V3{r.org.x - pos.x, r.org.y - pos.y, r.org.z - pos.z};
+        rr = r.dir;
+        if (flags & QR_DS_SHIFT)
+        {
+            if ((flags & QR_DS_TRM) != QR_DS_TRM_DIAG)
+            {
+                const float to[6] = {s.to[0], s.to[1], s.to[2], s.to[3], s.to[4], s.to[5]};
+                dd = xform_full(td, to, dd);
+                rr = xform_full(td, to, rr);
+            }
+            else
+            {
+                dd = xform_diag(td, dd);
+                rr = xform_diag(td, rr);
+            }
+        }
+    }
+    if (same) dd = r.oloc;
+    h.hit = ray_at(r.dir, r.org, h.t);
+    if (flags & QR_DS_SHIFT) h.loc = ray_at(rr, dd, h.t);
+    else h.loc = V3{h.hit.x - pos.x, h.hit.y - pos.y, h.hit.z - pos.z};
+    if (flags & QR_DS_APEX)
+    {
+        const float sci[4] = {s.sci[0], s.sci[1], s.sci[2], s.sci[3]};
+        const float scj[3] = {s.scj[0], s.scj[1], s.scj[2]};
+        float a_val, b_val, c_val;
+        const float d_val = quadric_abc(flags, sci, scj, rr, dd, a_val, b_val, c_val);
+        if (0.0f <= d_val && d_val < s.d_eps)
+        {
+            apex_snap(flags, sci, s.t_eps, dd, h.side, fbits(a_val) & SIGN, h.loc);
+        }
+    }
+    if ((flags & QR_DS_CLASS) == QR_DC_PLANE)
+    {
+        h.u = negif(sel(h.loc, amap(flags, 0)), asgn(flags, 0));
+        h.v = negif(sel(h.loc, amap(flags, 1)), asgn(flags, 1));
     }
     else
     {
@@ -876,17 +1022,19 @@ __device__ void hit_info(const Scene &sc, const Ray &r, Hit &h)
     }
 }
 
-
 /* surface normal in world space (PL 5669-5685, QD 6237-6281, TP 6415-6455,
  * transform 3273-3348) */
-__device__ V3 normal_at(const Scene &sc, const QC qr_surface &s, const Hit &h)
+__device__ V3 normal_at(const Scene &sc, const Hit &h)
 {
+    const QC qr_dev_surf &s = sc.hot[h.srf];
+    const uint32_t flags = s.flags;
+    const uint32_t kind = (flags >> QR_DS_NRM_BIT) & 3u;
     V3 n;
     const uint32_t ts = h.side ? SIGN : 0u;
-    if (s.nrm_kind == 1)
+    if (kind == 1)
     {
         V3 z = {0.0f, 0.0f, 0.0f};
-        put(z, s.amap[2], negif(fxor(1.0f, ts), s.asgn[2]));
+        put(z, amap(flags, 2), negif(fxor(1.0f, ts), asgn(flags, 2)));
         n = z;
     }
     else
@@ -895,7 +1043,7 @@ __device__ V3 normal_at(const Scene &sc, const QC qr_surface &s, const Hit &h)
         l.x = h.loc.x * s.sci[0];
         l.y = h.loc.y * s.sci[1];
         l.z = h.loc.z * s.sci[2];
-        if (s.nrm_kind == 2)
+        if (kind == 2)
         {
             l.x = l.x - s.scj[0];
             l.y = l.y - s.scj[1];
@@ -906,22 +1054,24 @@ __device__ V3 normal_at(const Scene &sc, const QC qr_surface &s, const Hit &h)
         float inv = fxor(rsq(rr), ts);
         n = V3{l.x * inv, l.y * inv, l.z * inv};
     }
-    if (s.trm == 0) return n;
+    if ((flags & QR_DS_TRM) == 0) return n;
 
-    const QC qr_surface &t = sc.srf[s.trnode];
-    float x = t.tc[0][0] * n.x;
-    float y = t.tc[1][1] * n.y;
-    float z = t.tc[2][2] * n.z;
+    const QC qr_dev_surf &t = sc.hot[s.trnode];
+    const uint32_t trm = t.flags & QR_DS_TRM;
+    float x = t.td[0] * n.x;
+    float y = t.td[1] * n.y;
+    float z = t.td[2] * n.z;
     bool renorm = true;
-    if (t.trm != 1)
+    if (trm != QR_DS_TRM_DIAG)
     {
-        x = x + t.tc[1][0] * n.y;
-        x = x + t.tc[2][0] * n.z;
-        y = y + t.tc[0][1] * n.x;
-        y = y + t.tc[2][1] * n.z;
-        z = z + t.tc[0][2] * n.x;
-        z = z + t.tc[1][2] * n.y;
-        renorm = t.trm != 2;
+        /* the transposed matrix: to holds 01 02 10 12 20 21 */
+        x = x + t.to[2] * n.y;
+        x = x + t.to[4] * n.z;
+        y = y + t.to[0] * n.x;
+        y = y + t.to[5] * n.z;
+        z = z + t.to[1] * n.x;
+        z = z + t.to[3] * n.y;
+        renorm = trm != QR_DS_TRM_ROT;
     }
     if (renorm)
     {

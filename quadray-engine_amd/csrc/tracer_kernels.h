@@ -28,7 +28,7 @@ typedef struct qr_dev_step
  * range (QR_DEV_STEP_BYTES times its index), which the walk adds to the
  * program's address as it is.  An element step carries what the walk needs
  * before it can load the surface record, so one scalar load of the step
- * starts it: skip is the record's byte offset in the surface table with the
+ * starts it: skip is the byte offset of its qr_dev_surf record with the
  * kind of its local box in the low two bits (records are 4-byte multiples),
  * and an element without a local box keeps its "last" (a transform node's
  * group end, else -1) in lo[0]'s bits.  Local boxes:
@@ -53,6 +53,129 @@ typedef struct qr_dev_step
 /* most records a surface table of the kernels holds (byte offsets fit an
  * int32) */
 #define QR_DEV_SURF_MAX ((int)(0x7fffffff / sizeof(qr_surface)))
+
+/* A surface as the walks read it: what one list element needs of its
+ * qr_surface record, in the order of use, with the small integers packed in
+ * one flag word.  The first 64 bytes (up to td) are one scalar load, which
+ * every element step issues at once; the rest is read by the surfaces that
+ * have clips or a full rotation.  Read from the 208-byte record, an element
+ * step was about fifteen scalar loads one after another, each for a control
+ * word that decided which came next, and a wave waited for each of them. */
+typedef struct qr_dev_surf
+{
+    float    pos[3];
+    uint32_t flags;             /* QR_DS_* */
+    float    sci[4];
+    float    scj[3];
+    float    d_eps, t_eps;
+    float    td[3];             /* diagonal of the inverse transform tc */
+    float    cmin[3], cmax[3];
+    float    to[6];             /* off its diagonal: 01 02 10 12 20 21 */
+    int32_t  clip_beg, clip_cnt;
+    int32_t  trnode;            /* record of the transform node, -1: none */
+    int32_t  pad;
+} qr_dev_surf;
+#define QR_DS_CLASS     0x7u            /* QR_DC_* */
+#define QR_DS_SHIFT     0x8u            /* traced in its node's frame */
+#define QR_DS_TRM       0x30u           /* any transform; bits: none, diagonal, */
+#define QR_DS_TRM_DIAG  0x10u           /* rotation, rotation and scale */
+#define QR_DS_TRM_ROT   0x20u
+#define QR_DS_NODE      0x40u           /* a transform node (an array) */
+#define QR_DS_APEX      0x80u
+#define QR_DS_APEX_TWO  0x100u          /* apex kind 2 (two planes) */
+#define QR_DS_CMIN_BIT  9               /* bit 9 + a: axis a has a min clip */
+#define QR_DS_CMAX_BIT  12
+#define QR_DS_AXIS_CLIP 0x7e00u
+#define QR_DS_CLIPS     0x8000u         /* has custom clippers */
+#define QR_DS_CLP_BIT   16              /* two bits: clp_kind 1, 2 or 3 */
+#define QR_DS_AMAP_BIT  18              /* two bits per local axis */
+#define QR_DS_ASGN_BIT  24              /* a bit per local axis */
+#define QR_DS_SHADOW_BIT 27             /* bit 27 + side: it casts shadows */
+#define QR_DS_NRM_BIT   29              /* two bits: nrm_kind 1, 2 or 3 */
+#define QR_DS_OWN_LIST  0x80000000u     /* rays leaving it walk a list of its own */
+/* classes: QR_SOLVE_* with the quadrics that need fewer operations apart.
+ * x - (+0) and x * 1 are x for every x, so those are the same roots. */
+#define QR_DC_PLANE     1
+#define QR_DC_QUADRIC   2
+#define QR_DC_TWOPLANE  3
+#define QR_DC_PURE      4               /* quadric, scj all +0 */
+#define QR_DC_SPHERE    5               /* pure, and sci[0..2] all 1 */
+
+/* does a surface side with these properties cast a shadow */
+static inline QR_HD int qr_casts_shadow(uint32_t p)
+{
+    if (p & QR_PROP_LIGHT) return 0;
+    if ((p & QR_PROP_TRANSP) && !(p & QR_PROP_REFRACT)) return 0;
+    return 1;
+}
+static inline QR_HD void qr_dev_surf_of(const qr_surface *r, int n_surf, qr_dev_surf *d)
+{
+    uint32_t f = r->solver >= QR_SOLVE_NONE && r->solver <= QR_SOLVE_QUADRIC
+                     ? (uint32_t)r->solver : (uint32_t)QR_DC_TWOPLANE;
+    if (f == QR_DC_QUADRIC)
+    {
+        int pure = 1, unit = 1;
+        for (int a = 0; a < 3; a++)
+        {
+            /* (+0 alone: x - (-0) is not x for x = -0) */
+            if (!(r->scj[a] == 0.0f && !__builtin_signbit(r->scj[a]))) pure = 0;
+            if (!(r->sci[a] == 1.0f)) unit = 0;
+        }
+        if (pure) f = unit ? QR_DC_SPHERE : QR_DC_PURE;
+    }
+    if (r->shift != 0) f |= QR_DS_SHIFT;
+    f |= r->trm == 0 ? 0u : r->trm == 1 ? QR_DS_TRM_DIAG : r->trm == 2 ? QR_DS_TRM_ROT
+                                                                       : QR_DS_TRM;
+    if (r->tag < 0) f |= QR_DS_NODE;
+    if (r->apex != 0) f |= QR_DS_APEX;
+    if (r->apex == 2) f |= QR_DS_APEX_TWO;
+    f |= ((uint32_t)r->cmin_on & 7u) << QR_DS_CMIN_BIT;
+    f |= ((uint32_t)r->cmax_on & 7u) << QR_DS_CMAX_BIT;
+    if (r->clip_cnt > 0) f |= QR_DS_CLIPS;
+    f |= (r->clp_kind == 1 || r->clp_kind == 2 ? (uint32_t)r->clp_kind : 3u) << QR_DS_CLP_BIT;
+    f |= (r->nrm_kind == 1 || r->nrm_kind == 2 ? (uint32_t)r->nrm_kind : 3u) << QR_DS_NRM_BIT;
+    for (int a = 0; a < 3; a++)
+    {
+        const uint32_t m = r->amap[a] == 0 ? 0u : r->amap[a] == 1 ? 1u : 2u;
+        f |= m << (QR_DS_AMAP_BIT + 2 * a);
+        if (r->asgn[a] != 0) f |= 1u << (QR_DS_ASGN_BIT + a);
+    }
+    for (int k = 0; k < 2; k++)
+    {
+        if (qr_casts_shadow(r->props[k])) f |= 1u << (QR_DS_SHADOW_BIT + k);
+    }
+    /* QuadRay gives a surface a nearest-hit list of its own for the rays
+     * leaving it when a side reflects or is not opaque
+     * (core/engine/engine.cpp:2180-2201) */
+    if (((r->props[0] | r->props[1]) & QR_PROP_REFLECT) != 0 ||
+        (r->props[0] & r->props[1] & QR_PROP_OPAQUE) == 0)
+    {
+        f |= QR_DS_OWN_LIST;
+    }
+    d->flags = f;
+    for (int a = 0; a < 3; a++)
+    {
+        d->pos[a] = r->pos[a];
+        d->sci[a] = r->sci[a];
+        d->scj[a] = r->scj[a];
+        d->td[a] = r->tc[a][a];
+        d->cmin[a] = r->cmin[a];
+        d->cmax[a] = r->cmax[a];
+    }
+    d->sci[3] = r->sci[3];
+    d->d_eps = r->d_eps;
+    d->t_eps = r->t_eps;
+    d->to[0] = r->tc[0][1];
+    d->to[1] = r->tc[0][2];
+    d->to[2] = r->tc[1][0];
+    d->to[3] = r->tc[1][2];
+    d->to[4] = r->tc[2][0];
+    d->to[5] = r->tc[2][1];
+    d->clip_beg = r->clip_beg;
+    d->clip_cnt = r->clip_cnt;
+    d->trnode = r->trnode >= 0 && r->trnode < n_surf ? r->trnode : -1;
+    d->pad = 0;
+}
 static inline QR_HD void qr_dev_box_step(qr_dev_step *d, int skip_index)
 {
     d->elem = -1;
@@ -72,7 +195,7 @@ static inline QR_HD void qr_dev_elem_step(qr_dev_step *d, int elem, int surf, in
                                           int local)
 {
     d->elem = elem;
-    d->skip = (int32_t)(surf * (int)sizeof(qr_surface)) | local;
+    d->skip = (int32_t)(surf * (int)sizeof(qr_dev_surf)) | local;
     if (local == QR_LOCAL_NONE)
     {
         for (int a = 0; a < 3; a++) d->lo[a] = d->hi[a] = 0.0f;
@@ -88,7 +211,7 @@ static inline QR_HD int qr_dev_step_local(const qr_dev_step *d)
 }
 static inline QR_HD int qr_dev_step_surf(const qr_dev_step *d)
 {
-    return (d->skip & ~3) / (int)sizeof(qr_surface);
+    return (d->skip & ~3) / (int)sizeof(qr_dev_surf);
 }
 /* the kind of local box the kernels give a list element whose program step
  * has one (a qr_cull_step with skip -2); groups 0: a program whose group
@@ -118,6 +241,7 @@ static inline QR_HD void qr_local_bounds(const qr_surface *srf, int surf, const 
 typedef struct qr_device_tables
 {
     qr_surface  *surfaces;
+    qr_dev_surf *hot;           /* the surfaces as the walks read them */
     qr_material *materials;
     qr_light    *lights;
     qr_clip     *clips;
@@ -130,16 +254,19 @@ typedef struct qr_device_tables
     float        cull_ref[4];   /* reference point of the world boxes */
 } qr_device_tables;
 
+/* hot[i] from srf[i] for every record, on the device */
+hipError_t qr_dev_surfaces(const qr_surface *srf, int n, qr_dev_surf *hot, hipStream_t stream);
+
 /* the device update stage's records (update.hip): every record of the
- * surface table, the planes' texture transforms in mat, and the surface
+ * surface table with its form for the walks (hot), the planes' texture transforms in mat, and the surface
  * list's element inputs of the culling programs, from the records' inputs
  * (fields.h); clips is the table's clip list; expect holds per element the
  * world and local flags the programs were built for, and an element that
  * differs sets *mismatch */
 struct qr_geom;
 hipError_t qr_update_records(const struct qr_geom *geoms, int n_rec, const qr_clip *clips,
-                             qr_surface *srf, qr_material *mat, struct qr_refit_elem *refit_in,
-                             const int32_t *expect, uint32_t *mismatch, hipStream_t stream);
+                             qr_surface *srf, qr_dev_surf *hot, qr_material *mat,
+                             struct qr_refit_elem *refit_in, const int32_t *expect, uint32_t *mismatch, hipStream_t stream);
 
 /* the device update stage's refit (update.hip): both programs' boxes (lo/hi
  * of every box step and of every element step with a local box) from the

@@ -294,7 +294,7 @@ k_pt_bounce(PtArgs a, int L)
         bool hit = false;
         if (live)
         {
-            const bool rev = r.origin < 0 || own_list(a.sc.srf[r.origin]);
+            const bool rev = r.origin < 0 || own_list(a.sc, r.origin);
             hit = walk<false>(a.sc, r, h, rev);
         }
         bool emit = false;
@@ -309,7 +309,7 @@ k_pt_bounce(PtArgs a, int L)
             const QC qr_surface &s = a.sc.srf[h.srf];
             const uint32_t props = s.props[h.side];
             const QC qr_material &m = a.sc.mat[s.mat[h.side]];
-            const V3 nrm = normal_at(a.sc, s, h);
+            const V3 nrm = normal_at(a.sc, h);
             V3 tex = texel_color(a.sc, m, props, h);
 
             const uint32_t pass = sid / a.n0;

@@ -491,13 +491,13 @@ __device__ __forceinline__ void nearest(const QC Frame &a, int L, uint32_t i,
     Hit h;
     h.srf = -1;
     bool hit = false;
-    if (valid) hit = walk<false>(sc, r, h);
+    if (valid) hit = walk<false, !L0>(sc, r, h);
 
     V3 nrm = V3{0.0f, 0.0f, 0.0f};
     if (hit)
     {
         hit_info(sc, r, h);
-        nrm = normal_at(sc, sc.srf[h.srf], h);
+        nrm = normal_at(sc, h);
         cur.na[i] = make_float4(h.hit.x, h.hit.y, h.hit.z,
                                 __int_as_float((h.srf << 1) | h.side));
         cur.nb[i] = make_float4(h.loc.x, h.loc.y, h.loc.z, h.u);

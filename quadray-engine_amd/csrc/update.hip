@@ -124,7 +124,8 @@ __global__ void __launch_bounds__(RF_WG) k_boxes(qr_dev_step *prog0, int n0, qr_
  * longer fits: the host rebuilds them) */
 __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
                                                  const qr_clip *clips, qr_surface *srf,
-                                                 qr_material *mat, qr_refit_elem *refit_in,
+                                                 qr_dev_surf *hot, qr_material *mat,
+                                                 qr_refit_elem *refit_in,
                                                  const int32_t *expect, uint32_t *mismatch)
 {
     const int r = blockIdx.x * 64 + threadIdx.x;
@@ -135,6 +136,7 @@ __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
         qr_surface out;
         qf_array_record(g, out);
         srf[r] = out;
+        qr_dev_surf_of(&out, n_rec, &hot[r]);
         if (g.elem >= 0)
         {
             qr_refit_elem z;
@@ -151,6 +153,7 @@ __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
     qr_surface out;
     qf_surface_record(g, sci, scj, bmin, bmax, cmin, cmax, out);
     srf[r] = out;
+    qr_dev_surf_of(&out, n_rec, &hot[r]);
     if (g.tag == RT_TAG_PLANE)
     {
         for (int side = 0; side < 2; side++)
@@ -176,17 +179,32 @@ __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
     }
 }
 
+/* the walks' form of records that came from the host */
+__global__ void __launch_bounds__(64) k_surfaces(const qr_surface *srf, int n, qr_dev_surf *hot)
+{
+    const int r = blockIdx.x * 64 + threadIdx.x;
+    if (r < n) qr_dev_surf_of(&srf[r], n, &hot[r]);
+}
+
 }  /* namespace */
 
+hipError_t qr_dev_surfaces(const qr_surface *srf, int n, qr_dev_surf *hot, hipStream_t stream)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_surfaces, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, stream, srf, n,
+                       hot);
+    return hipGetLastError();
+}
+
 hipError_t qr_update_records(const qr_geom *geoms, int n_rec, const qr_clip *clips,
-                             qr_surface *srf, qr_material *mat, qr_refit_elem *refit_in,
-                             const int32_t *expect, uint32_t *mismatch, hipStream_t stream)
+                             qr_surface *srf, qr_dev_surf *hot, qr_material *mat,
+                             qr_refit_elem *refit_in, const int32_t *expect, uint32_t *mismatch, hipStream_t stream)
 {
     if (n_rec <= 0) return hipSuccess;
     /* one wave per workgroup: a record's work is a long serial chain, so
      * the records spread over as many compute units as they can */
     hipLaunchKernelGGL(k_records, dim3((unsigned)((n_rec + 63) / 64)), dim3(64), 0, stream,
-                       geoms, n_rec, clips, srf, mat, refit_in, expect, mismatch);
+                       geoms, n_rec, clips, srf, hot, mat, refit_in, expect, mismatch);
     return hipGetLastError();
 }
 

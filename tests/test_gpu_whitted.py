@@ -9,6 +9,7 @@ fp32 root selection is ill-conditioned)."""
 import numpy as np
 import pytest
 
+import qr_oracle
 import qrhip
 from helpers import (GoldenTables, HostScene, assert_frame_exact, channels, frame_stats,
                      golden_camera_cases, golden_cases, golden_frame, golden_table_cases,
@@ -313,3 +314,29 @@ def test_gpu_texture_files_render_as_texel_arrays(device, tmp_path):
         qrhip.set_data_path("../")
     assert len(list((tmp_path / "data" / "textures").iterdir())) > 0
     assert np.array_equal(frames[0], frames[1])
+
+
+@pytest.mark.parametrize("config,seed", [(9, 3), (2, 5)])
+@pytest.mark.parametrize("d_eps,zero", [(0.0, 0.0), (1.0e-30, -0.0), (1.0, 0.0),
+                                        (1.2621774e-29, -0.0)])
+def test_gpu_root_forms(path_dev, config, seed, d_eps, zero):
+    """Each way the walks form a surface's roots, on caller tables: no
+    near-zero discriminants, thresholds below and at the smallest value the
+    short square root takes, many of them, and linear terms of either zero
+    (only +0 leaves them out); bit for bit the oracle's frame."""
+    hs = HostScene(config, seed, 97, 61, 1, 3)
+    try:
+        snap = qrhip.tables_snapshot(hs.tables, hs.fd)
+    finally:
+        hs.close()
+    t = qrhip.TablesFromSnapshot(snap)
+    for i in range(t.tables.n_surf):
+        s = t.tables.surfaces[i]
+        s.d_eps = d_eps
+        for a in range(3):
+            if s.scj[a] == 0.0:
+                s.scj[a] = zero
+    want, ids_o, flags, _, _ = qr_oracle.render(t.ptr, t.fd, want_ids=True)
+    got, ids = path_dev.render_tables(t.ptr, t.fd, want_ids=True)
+    assert_frame_exact(got, want, f"config {config} d_eps {d_eps} zero {zero}")
+    assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
