@@ -98,6 +98,13 @@ struct PtArgs
     uint32_t      *cnt;                 /* CNT_N counters */
 };
 
+/* bits of a wave mask below this lane */
+__device__ __forceinline__ uint32_t below(uint64_t m)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 /* next number of the slot's LCG as a float in [0, 1): top 24 bits over 2^24
  * (GET_RANDOM_F tracer.cpp:1949-1980, LCG24 tracer.h:58) */
 __device__ __forceinline__ float pt_random(uint32_t &st)
@@ -165,34 +172,45 @@ __device__ __forceinline__ bool chunk_pixel(const PtArgs &a, uint32_t j, int &x,
     return x < a.fd.x_res && y < a.fd.y_res;
 }
 
-/* a lane's first slot for "cnt" (0..3) entries of one queue: the wave's
- * prefix from two ballots of the count's bits, the workgroup's from the
- * waves' totals in LDS, one global atomic per workgroup.  Every thread of
- * the workgroup calls it. */
-__device__ __forceinline__ uint32_t wg_append(uint32_t cnt, uint32_t *counter,
-                                              uint32_t *sh_tot, uint32_t *sh_base)
+/* a lane's slot for a contribution (emit) and its first slot for "kids"
+ * (0..3) rays: the wave's prefixes from ballots, the workgroup's from the
+ * waves' totals in LDS, one global atomic per workgroup and queue, made by
+ * two threads side by side.  Every thread of the workgroup calls it; the
+ * totals alternate between two buffers ("odd"), so a call need not wait for
+ * the previous one's readers. */
+struct Append
+{
+    uint32_t tot[2][2][WAVES];      /* [odd][queue][wave] */
+    uint32_t base[2][2];
+};
+
+__device__ __forceinline__ void wg_append(Append &sh, int odd, bool emit, uint32_t kids,
+                                          uint32_t *cnt_emit, uint32_t *cnt_kids,
+                                          uint32_t &at_emit, uint32_t &at_kids)
 {
     const int wv = threadIdx.x >> 6;
-    const int lane = __lane_id();
-    const uint64_t b0 = __ballot(cnt & 1u), b1 = __ballot((cnt >> 1) & 1u);
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t pre = (uint32_t)__popcll(b0 & below) + 2u * (uint32_t)__popcll(b1 & below);
-    __syncthreads();                    /* the previous call's totals are read */
-    if (lane == 0) sh_tot[wv] = (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1);
+    const uint64_t be = lanes(emit), b0 = lanes((kids & 1u) != 0), b1 = lanes((kids & 2u) != 0);
+    if (__lane_id() == 0)
+    {
+        sh.tot[odd][0][wv] = (uint32_t)__popcll(be);
+        sh.tot[odd][1][wv] = (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1);
+    }
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (threadIdx.x < 2)
     {
         uint32_t run = 0;
         for (int v = 0; v < WAVES; v++)
         {
-            const uint32_t t = sh_tot[v];
-            sh_tot[v] = run;
+            const uint32_t t = sh.tot[odd][threadIdx.x][v];
+            sh.tot[odd][threadIdx.x][v] = run;
             run += t;
         }
-        *sh_base = run != 0 ? atomicAdd(counter, run) : 0u;
+        sh.base[odd][threadIdx.x] = run != 0 ? atomicAdd(threadIdx.x == 0 ? cnt_emit : cnt_kids,
+                                                         run) : 0u;
     }
     __syncthreads();
-    return *sh_base + sh_tot[wv] + pre;
+    at_emit = sh.base[odd][0] + sh.tot[odd][0][wv] + below(be);
+    at_kids = sh.base[odd][1] + sh.tot[odd][1][wv] + below(b0) + 2u * below(b1);
 }
 
 __device__ __forceinline__ void put_ray(const PtArgs &a, int out, uint32_t idx, const Hit &h,
@@ -219,8 +237,8 @@ __device__ __forceinline__ void put_ray(const PtArgs &a, int out, uint32_t idx, 
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(6, 6)))
 k_pt_bounce(PtArgs a, int L)
 {
-    __shared__ uint32_t sh_tot[WAVES];
-    __shared__ uint32_t sh_base;
+    __shared__ Append sh;
+    int odd = 0;
     /* an overflowed queue holds only its first cap_q rays */
     const uint32_t n = L == 0 ? a.n0 * a.passes : min(a.cnt[L], a.cap_q);
     const int in = L & 1, out = (L + 1) & 1;
@@ -312,13 +330,20 @@ k_pt_bounce(PtArgs a, int L)
             const V3 nrm = normal_at(a.sc, h);
             V3 tex = texel_color(a.sc, m, props, h);
 
-            const uint32_t pass = sid / a.n0;
-            const float pts_o = 1.0f / (a.pts_c0 + (float)pass);
-            float c;
-            c = m.col[0] * pts_o; col.x = c * mul.x;
-            c = m.col[1] * pts_o; col.y = c * mul.y;
-            c = m.col[2] * pts_o; col.z = c * mul.z;
-            emit = col.x != 0.0f || col.y != 0.0f || col.z != 0.0f;
+            /* emission, of the few surfaces that have one (a throughput that
+             * is not finite turns no emission into NaN) */
+            const V3 em = V3{m.col[0], m.col[1], m.col[2]};
+            const float fin = mul.x * 0.0f + mul.y * 0.0f + mul.z * 0.0f;
+            if (em.x != 0.0f || em.y != 0.0f || em.z != 0.0f || !(fin == 0.0f))
+            {
+                const uint32_t pass = sid / a.n0;
+                const float pts_o = 1.0f / (a.pts_c0 + (float)pass);
+                float c;
+                c = em.x * pts_o; col.x = c * mul.x;
+                c = em.y * pts_o; col.y = c * mul.y;
+                c = em.z * pts_o; col.z = c * mul.z;
+                emit = col.x != 0.0f || col.y != 0.0f || col.z != 0.0f;
+            }
 
             if (props & QR_PROP_DIFFUSE)
             {
@@ -351,9 +376,11 @@ k_pt_bounce(PtArgs a, int L)
                     v.x = nrm.y * u.z - nrm.z * u.y;
                     v.y = nrm.z * u.x - nrm.x * u.z;
                     v.z = nrm.x * u.y - nrm.y * u.x;
+                    /* r1 is a multiple of 2^-24 below 1: 0 or in
+                     * sqrt_mid's range, and so is 1 - r1 */
                     const float r1 = pt_random(st);
-                    const float sn = sqrtf(r1);
-                    const float cs = sqrtf(1.0f - r1);
+                    const float sn = sqrt_mid(r1);
+                    const float cs = sqrt_mid(1.0f - r1);
                     const float r2 = pt_random(st);
                     float phi = (r2 + r2) * 3.14159265358979323846f;
                     phi = phi - 3.14159265358979323846f;
@@ -381,8 +408,9 @@ k_pt_bounce(PtArgs a, int L)
                 qv = qv * 0.5f;
                 const float pr = 0.25f + qv;
                 const bool pick_tr = rr >= pr;
-                t.c_trn = pick_tr ? t.c_trn / (1.0f - pr) : 0.0f;
-                t.c_rfl = pick_tr ? 0.0f : t.c_rfl / pr;
+                const float c = (pick_tr ? t.c_trn : t.c_rfl) / (pick_tr ? 1.0f - pr : pr);
+                t.c_trn = pick_tr ? c : 0.0f;
+                t.c_rfl = pick_tr ? 0.0f : c;
                 t.tr = t.tr && pick_tr;
                 t.rf = t.rf && !pick_tr;
             }
@@ -401,7 +429,10 @@ k_pt_bounce(PtArgs a, int L)
         }
 
         /* the sample's contribution, linked into its list */
-        const uint32_t ci = wg_append(emit ? 1u : 0u, &a.cnt[CNT_CONTRIB], sh_tot, &sh_base);
+        const uint32_t nk = (uint32_t)__popc(kids);
+        uint32_t ci, at;
+        wg_append(sh, odd, emit, nk, &a.cnt[CNT_CONTRIB], &a.cnt[L + 1], ci, at);
+        odd ^= 1;
         if (emit)
         {
             if (ci < a.cap_c)
@@ -418,8 +449,6 @@ k_pt_bounce(PtArgs a, int L)
         /* the children, compacted into the next bounce's queue; every slot
          * below the capacity is written, so the next bounce reads only rays
          * of this run even after an overflow */
-        const uint32_t nk = (uint32_t)__popc(kids);
-        uint32_t at = wg_append(nk, &a.cnt[L + 1], sh_tot, &sh_base);
         if (nk != 0 && (uint64_t)at + nk > a.cap_q) a.cnt[CNT_OVERFLOW] = 1u;
         if ((kids & 1u) && at < a.cap_q)
             put_ray(a, out, at, h, r_dir, h.side, st, r_mul, key * 4u + KEY_RF, sid);
