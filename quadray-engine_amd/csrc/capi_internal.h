@@ -543,7 +543,9 @@ struct qrhip_scene
     size_t       pt_slots = 0;
     bool         pt_reset = true;      /* seeds and planes to (re)start */
     int          pt_fsaa = -1;         /* AA mode the planes were made with */
-    uint32_t    *staging = nullptr;    /* pinned host copy of dframe */
+    uint32_t    *staging = nullptr;    /* pinned host copy of dframe: the frame
+                                          itself when the scene owns it and
+                                          its rows have no gap */
     hipEvent_t   ev0 = nullptr, ev1 = nullptr;
 };
 

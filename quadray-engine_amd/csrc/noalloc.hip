@@ -236,9 +236,15 @@ int qrhip_render_tables_noalloc(qrhip_dev *dev, const qr_scene_tables *tab,
     int32_t *dids = ids != nullptr ? (int32_t *)(base + part[11].off) : nullptr;
     HIP_TRY(qr_launch_whitted(&t, &d, dfr, dids, st));
 
-    /* rows to the caller's frame at its pitch (negative: rows run backwards) */
+    /* rows to the caller's frame at its pitch (negative: rows run
+     * backwards); with no gap between them the frame is one copy (a copy of
+     * 360 rows to pageable memory took 1.7 ms, one of 0.9 MB 0.1 ms) */
     const size_t row = sizeof(uint32_t) * (size_t)fd->x_res;
-    if (fd->x_row > 0)
+    if (fd->x_row == fd->x_res)
+    {
+        HIP_TRY(hipMemcpyAsync(frame, dfr, row * (size_t)fd->y_res, hipMemcpyDeviceToHost, st));
+    }
+    else if (fd->x_row > 0)
     {
         HIP_TRY(hipMemcpy2DAsync(frame, sizeof(uint32_t) * (size_t)fd->x_row, dfr, row, row,
                                  (size_t)fd->y_res, hipMemcpyDeviceToHost, st));

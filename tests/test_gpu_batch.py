@@ -283,3 +283,42 @@ def test_batch_at_benchmark_shape_against_oracle(device):
         for r, px in rows.items():
             assert np.array_equal(got[k][r], px), f"frame {k} {bc.keys[k]} row {r}"
     print("batch: sampled rows equal the oracle", flush=True)
+
+
+@pytest.mark.parametrize("sizes", [[(3, 5)], [(1, 1), (1031, 517), (2, 3)],
+                                   [(1920, 1080), (33, 17), (640, 360), (1021, 769)],
+                                   [(4099, 2053), (17, 9), (4096, 2048)]])
+def test_batch_download_parts(device, sizes):
+    """Frames downloaded together, in one part, in parts cut inside frames,
+    and in more than one round of pinned memory, equal the scenes' own; so
+    does one frame downloaded alone, and the frame of a scene with padded
+    rows."""
+    w = qrhip.Workload(1, 6)
+    scenes = [qrhip.Scene(device, w.ptr, 64, 64)]
+    b = qrhip.Batch(device)
+    try:
+        scenes[0].update(0)
+        b.set([(scenes[0], x, y, 0, 1) for x, y in sizes])
+        got = b.render(qrhip.BATCH_DIRECT)
+        last = len(sizes) - 1
+        b.bufs[last][:] = 0
+        qrhip.check(qrhip.lib().qrhip_batch_download(b.h, last))
+        assert np.array_equal(b.bufs[last], got[last])
+    finally:
+        b.destroy()
+        for s in scenes:
+            s.destroy()
+        w.close()
+    device.set_fsaa(0)
+    for (x, y), f in zip(sizes, got):
+        for pad in (0, 3):
+            w = qrhip.Workload(1, 6)
+            s = qrhip.Scene(device, w.ptr, x, y, x_row=x + pad)
+            try:
+                s.set_depth(1)
+                assert not s.frame().any()      # blank before the first render
+                want = s.render(0)
+            finally:
+                s.destroy()
+                w.close()
+            assert np.array_equal(f, want), f"frame {x}x{y} pad {pad}"
