@@ -32,29 +32,6 @@ int hip_fail(hipError_t e, const char *what)
     return fail(QRHIP_E_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-/* initial seed plane: the low 32 bits of a 48-bit LCG chain started at 1,
- * one value per framebuffer sample slot in QuadRay's order, slot
- * (y * |x_row| + x) * samples + k (rt_Scene::reset_pseed,
- * core/engine/engine.cpp:3719-3740); here gathered to (y * x_res + x) *
- * samples + k */
-void pt_seed_plane(std::vector<uint32_t> &out, int x_res, int y_res, int x_row, int ns)
-{
-    const int ar = x_row < 0 ? -x_row : x_row;
-    out.assign((size_t)x_res * y_res * ns, 0u);
-    uint64_t st = 1;
-    for (int y = 0; y < y_res; y++)
-    {
-        for (int x = 0; x < ar; x++)
-        {
-            for (int j = 0; j < ns; j++)
-            {
-                st = (st * 25214903917ull + 11ull) & 0x0000FFFFFFFFFFFFull;
-                if (x < x_res) out[((size_t)y * x_res + x) * ns + j] = (uint32_t)st;
-            }
-        }
-    }
-}
-
 /* enqueue one Whitted frame on the device's chosen path */
 hipError_t launch_frame(const qrhip_dev *d, qr_wf_state *wf, const qr_device_tables *t,
                         const qr_frame_desc *fd, uint32_t *frame, int32_t *ids)
@@ -547,16 +524,10 @@ int qrhip_scene_launch(qrhip_scene *s)
         if (s->pt_fsaa != s->fd.fsaa) s->pt_reset = true;
         if (s->pt_reset || s->pt_slots != slots)
         {
-            std::vector<uint32_t> seeds;
-            pt_seed_plane(seeds, s->x_res, s->y_res, s->x_row, ns);
-            std::vector<float> zero(3 * slots, 0.0f);
             HIP_TRY(s->pt_seeds.reserve(sizeof(uint32_t) * slots));
             HIP_TRY(s->pt_planes.reserve(sizeof(float) * 3 * slots));
-            HIP_TRY(hipMemcpyAsync(s->pt_seeds.ptr, seeds.data(), sizeof(uint32_t) * slots,
-                                   hipMemcpyHostToDevice, s->dev->stream));
-            HIP_TRY(hipMemcpyAsync(s->pt_planes.ptr, zero.data(), sizeof(float) * 3 * slots,
-                                   hipMemcpyHostToDevice, s->dev->stream));
-            HIP_TRY(hipStreamSynchronize(s->dev->stream));
+            HIP_TRY(qr_pt_start((float *)s->pt_planes.ptr, (uint32_t *)s->pt_seeds.ptr, s->x_res,
+                                s->y_res, s->x_row, s->fd.fsaa, s->dev->stream));
             s->pts_c = 0.0f;
             s->pt_slots = slots;
             s->pt_reset = false;
@@ -923,9 +894,24 @@ int qrhip_pt_seed_plane(int x_res, int y_res, int x_row, int fsaa, uint32_t *see
     {
         return fail(QRHIP_E_ARG, "bad argument");
     }
-    std::vector<uint32_t> v;
-    pt_seed_plane(v, x_res, y_res, x_row, fsaa == 2 ? 4 : fsaa == 1 ? 2 : 1);
-    memcpy(seeds, v.data(), v.size() * sizeof(uint32_t));
+    /* the low 32 bits of a 48-bit LCG chain started at 1, one value per
+     * framebuffer sample slot in QuadRay's order, slot (y * |x_row| + x) *
+     * samples + k (rt_Scene::reset_pseed, core/engine/engine.cpp:3719-3740);
+     * here gathered to (y * x_res + x) * samples + k */
+    const int ns = fsaa == 2 ? 4 : fsaa == 1 ? 2 : 1;
+    const int ar = x_row < 0 ? -x_row : x_row;
+    uint64_t st = 1;
+    for (int y = 0; y < y_res; y++)
+    {
+        for (int x = 0; x < ar; x++)
+        {
+            for (int j = 0; j < ns; j++)
+            {
+                st = (st * 25214903917ull + 11ull) & 0x0000FFFFFFFFFFFFull;
+                if (x < x_res) seeds[((size_t)y * x_res + x) * ns + j] = (uint32_t)st;
+            }
+        }
+    }
     return QRHIP_OK;
 }
 

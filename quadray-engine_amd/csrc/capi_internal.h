@@ -557,10 +557,6 @@ inline bool has_gpu(const qrhip_dev *d)
     return d != nullptr && d->ordinal >= 0;
 }
 
-/* a frame's initial path-tracer seed plane, slot (y * x_res + x) * ns + k,
- * from QuadRay's seed chain over rows of |x_row| pixels */
-void pt_seed_plane(std::vector<uint32_t> &out, int x_res, int y_res, int x_row, int ns);
-
 /* every table index the kernels follow stays inside its table, and the
  * frame description is in range (QRHIP_OK, or the failure reported) */
 int validate_tables(const qr_scene_tables *tab, const qr_frame_desc *fd);

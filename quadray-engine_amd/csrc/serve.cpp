@@ -58,8 +58,6 @@ struct Slot
     DevBuf    planes, seeds;            /* path tracer */
     uint32_t *host = nullptr;           /* pinned: frame copy back */
     size_t    host_cap = 0;
-    uint32_t *staged = nullptr;         /* pinned: seed plane upload */
-    size_t    staged_cap = 0;
     bool      busy = false;
 };
 
@@ -297,22 +295,12 @@ hipError_t qrhip_server::admit_one(Req *q)
 
     if (pt)
     {
-        /* the seed plane and cleared colour planes; the pinned staging copy
-         * stays untouched until the slot is reassigned */
+        /* the seed plane and cleared colour planes */
         const size_t slots_n = px * (size_t)ns;
-        std::vector<uint32_t> seeds;
-        pt_seed_plane(seeds, q->r.x_res, q->r.y_res, q->r.x_res, ns);
-        if ((e = pinned_reserve(sl.staged, sl.staged_cap, slots_n)) != hipSuccess) return e;
-        memcpy(sl.staged, seeds.data(), sizeof(uint32_t) * slots_n);
         if ((e = sl.seeds.reserve(sizeof(uint32_t) * slots_n)) != hipSuccess) return e;
         if ((e = sl.planes.reserve(sizeof(float) * 3 * slots_n)) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(sl.seeds.ptr, sl.staged, sizeof(uint32_t) * slots_n,
-                                hipMemcpyHostToDevice, stream)) != hipSuccess)
-        {
-            return e;
-        }
-        if ((e = hipMemsetAsync(sl.planes.ptr, 0, sizeof(float) * 3 * slots_n, stream)) !=
-            hipSuccess)
+        if ((e = qr_pt_start((float *)sl.planes.ptr, (uint32_t *)sl.seeds.ptr, q->r.x_res,
+                             q->r.y_res, q->r.x_res, q->r.fsaa, stream)) != hipSuccess)
         {
             return e;
         }
@@ -910,7 +898,6 @@ int qrhip_server_destroy(qrhip_server *s)
         sl.planes.release();
         sl.seeds.release();
         if (sl.host != nullptr) (void)hipHostFree(sl.host);
-        if (sl.staged != nullptr) (void)hipHostFree(sl.staged);
     }
     if (s->copied != nullptr) (void)hipEventDestroy(s->copied);
     (void)hipStreamDestroy(s->stream);

@@ -289,6 +289,11 @@ hipError_t qr_launch_whitted(const qr_device_tables *t, const qr_frame_desc *fd,
 typedef struct qr_pt_state qr_pt_state;
 hipError_t qr_pt_create(qr_pt_state **out);
 void       qr_pt_destroy(qr_pt_state *s);
+/* a path-traced frame's start: cleared planes (3 x slots floats) and the
+ * initial seed plane of a frame of x_res x y_res with rows of |x_row| pixels,
+ * in the slot order below (at most 2^32 - 1 slots) */
+hipError_t qr_pt_start(float *planes, uint32_t *seeds, int x_res, int y_res, int x_row,
+                       int fsaa, hipStream_t stream);
 /* "passes" passes over the chunk of 8x8-pixel tiles tile0 .. tile0 +
  * ntiles - 1 (ntiles 0: all), fd->pts_c counting the first: planes (red,
  * green, blue running means, 3 x slots floats) and seeds (one per slot),

@@ -461,6 +461,41 @@ k_pt_bounce(PtArgs a, int L)
     }
 }
 
+/* jumps of the seed chain: 2^i of its steps are x * mul[i] + add[i] */
+struct SeedJumps
+{
+    uint64_t mul[48], add[48];
+};
+
+/* a frame's cleared colour planes and initial seed plane: the low 32 bits of
+ * a 48-bit LCG chain started at 1, one value per framebuffer sample slot of
+ * a frame with rows of "row" pixels (rt_Scene::reset_pseed,
+ * core/engine/engine.cpp:3719-3740), gathered to slot (y * x_res + x) *
+ * samples + k.  The chain is serial, so each work-item jumps to its slot's
+ * number in as many steps as it has bits.  Bound by its stores: 20 us for
+ * 1280x720, against 1.9 ms for the host's chain, its copies and a wait. */
+__global__ void __launch_bounds__(WG) k_pt_start(SeedJumps j, float *planes, uint32_t *seeds,
+                                                 uint32_t slots, uint32_t x_res, uint64_t row,
+                                                 uint32_t ns)
+{
+    for (uint64_t at = blockIdx.x * (uint64_t)WG + threadIdx.x; at < slots;
+         at += gridDim.x * (uint64_t)WG)
+    {
+        const uint32_t i = (uint32_t)at;
+        const uint32_t px = i / ns, y = px / x_res;
+        uint64_t n = ((uint64_t)y * row + (px - y * x_res)) * ns + (i - px * ns) + 1u;
+        uint64_t st = 1;
+        for (int b = 0; n != 0; b++, n >>= 1)
+        {
+            if (n & 1u) st = st * j.mul[b] + j.add[b];
+        }
+        seeds[i] = (uint32_t)st;
+        planes[i] = 0.0f;
+        planes[(size_t)slots + i] = 0.0f;
+        planes[2 * (size_t)slots + i] = 0.0f;
+    }
+}
+
 /* start of a run: counters and the samples' list heads cleared (a fill
  * kernel rather than a memset, so the launch can be captured) */
 __global__ void __launch_bounds__(WG) k_pt_reset(PtArgs a)
@@ -730,6 +765,29 @@ void qr_pt_destroy(qr_pt_state *s)
 uint32_t qr_pt_tiles(int x_res, int y_res)
 {
     return (uint32_t)((x_res + PT_TILE - 1) / PT_TILE) * (uint32_t)((y_res + PT_TILE - 1) / PT_TILE);
+}
+
+hipError_t qr_pt_start(float *planes, uint32_t *seeds, int x_res, int y_res, int x_row,
+                       int fsaa, hipStream_t stream)
+{
+    const int ns = fsaa == 2 ? 4 : fsaa == 1 ? 2 : 1;
+    const uint64_t slots = (uint64_t)x_res * (uint64_t)y_res * (uint64_t)ns;
+    if (x_res <= 0 || y_res <= 0 || slots > 0xFFFFFFFFull) return hipErrorInvalidValue;
+    SeedJumps j;
+    j.mul[0] = 25214903917ull;
+    j.add[0] = 11ull;
+    for (int i = 1; i < 48; i++)
+    {
+        /* (the chain is modulo 2^48; the low bits of a product do not
+         * depend on the high ones) */
+        j.mul[i] = j.mul[i - 1] * j.mul[i - 1];
+        j.add[i] = j.add[i - 1] * (j.mul[i - 1] + 1ull);
+    }
+    const uint64_t row = x_row < 0 ? (uint64_t)(-(int64_t)x_row) : (uint64_t)x_row;
+    const unsigned g = (unsigned)std::min<uint64_t>((slots + WG - 1) / WG, 16384u);
+    hipLaunchKernelGGL(k_pt_start, dim3(g), dim3(WG), 0, stream, j, planes, seeds,
+                       (uint32_t)slots, (uint32_t)x_res, row, (uint32_t)ns);
+    return hipGetLastError();
 }
 
 hipError_t qr_pt_launch(qr_pt_state *s, const qr_device_tables *t, const qr_frame_desc *fd,

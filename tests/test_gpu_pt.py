@@ -97,3 +97,34 @@ def test_gpu_pt_passes_in_one_launch(device, config, seed, x, y, fsaa, depth):
     finally:
         hs.close()
     assert np.array_equal(frames[0], fw)
+
+
+@pytest.mark.parametrize("x,y,fsaa,x_row", [(1, 1, 0, 1), (17, 3, 2, 17), (65, 33, 1, 70),
+                                            (64, 48, 2, -64), (257, 131, 0, -300),
+                                            (513, 257, 2, 520)])
+def test_gpu_pt_scene_seeds(device, x, y, fsaa, x_row):
+    """The planes and seeds that a scene's path tracer starts from on the
+    device, for every AA mode, row pitch and direction: one pass of the scene
+    equals one pass over its tables from the host's seed plane, and so does
+    the first pass after the path tracer was switched off and on again."""
+    device.set_fsaa(fsaa)
+    w = qrhip.Workload(3, 31)
+    s = qrhip.Scene(device, w.ptr, x, y, x_row=x_row)
+    try:
+        s.set_depth(3)
+        s.set_pton(1)
+        got = s.render(0)
+        s.render(0)
+        s.set_pton(0)
+        s.set_pton(1)
+        again = s.render(0)
+        tables, fd = s.tables()
+        fd.pt_on, fd.pts_c, fd.x_row = 1, 1.0, x
+        planes = np.zeros((3, x * y * (1, 2, 4)[fsaa]), dtype=np.float32)
+        want = device.render_tables_pt(tables, fd, planes,
+                                       qrhip.pt_seed_plane(x, y, x_row, fsaa))
+    finally:
+        s.destroy()
+        w.close()
+    assert np.array_equal(got, want)
+    assert np.array_equal(again, want)
