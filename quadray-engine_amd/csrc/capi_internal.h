@@ -227,8 +227,8 @@ inline ProgramInputs program_inputs(const qr::Engine &eng)
 struct DevTables
 {
     DevBuf srf, hot, mat, lgt, clp, elem, tex, step, step_any, refit_in, refit_box;
-    DevBuf geom, expect, flag;      /* the device update stage's inputs */
-    uint32_t *flag_host = nullptr;  /* pinned copy of flag */
+    DevBuf geom, expect;            /* the device update stage's inputs */
+    uint32_t *flag_host = nullptr;  /* pinned: set by the device's kernels */
     uint64_t expect_build = 0;      /* the build "expect" holds the flags of */
     Stager stage;
     std::vector<uint8_t> sent[8];   /* what each table's buffer holds now */
@@ -387,6 +387,16 @@ struct DevTables
         t.n_clip = h.n_clip;
         t.n_elem = h.n_elem;
         t.n_texel = h.n_texel;
+        t.spawns = 0;
+        for (int i = 0; i < h.n_surf; i++)
+        {
+            const qr_surface &s = h.surfaces[i];
+            if (s.solver != QR_SOLVE_NONE &&
+                (qr_side_spawns(s.props[0]) || qr_side_spawns(s.props[1])))
+            {
+                t.spawns = 1;
+            }
+        }
         return hipSuccess;
     }
     void release()
@@ -394,7 +404,7 @@ struct DevTables
         srf.release(); hot.release(); mat.release(); lgt.release();
         clp.release(); elem.release(); tex.release(); step.release();
         step_any.release(); refit_in.release(); refit_box.release();
-        geom.release(); expect.release(); flag.release();
+        geom.release(); expect.release();
         if (flag_host != nullptr) (void)hipHostFree(flag_host);
         flag_host = nullptr;
         stage.release();
@@ -432,7 +442,6 @@ struct DevTables
         const size_t ebytes = sizeof(int32_t) * 2 * (size_t)n_elem;
         if ((e = geom.reserve(gbytes)) != hipSuccess) return e;
         if ((e = expect.reserve(ebytes)) != hipSuccess) return e;
-        if ((e = flag.reserve(sizeof(uint32_t))) != hipSuccess) return e;
         if ((e = refit_in.reserve(sizeof(qr_refit_elem) * (size_t)n_elem)) != hipSuccess) return e;
         if ((e = refit_box.reserve(sizeof(float) * 8 * (size_t)n_elem)) != hipSuccess) return e;
         if (flag_host == nullptr &&
@@ -456,13 +465,11 @@ struct DevTables
         const size_t lbytes = sizeof(qr_light) * (size_t)h.n_lgt;
         const bool send_lgt = lbytes > 0 && (sent[4].size() != lbytes ||
                                              memcmp(sent[4].data(), h.lights, lbytes) != 0);
-        const uint32_t zero = 0u;
-        size_t total = ((gbytes + 255) & ~(size_t)255) + 256;
+        size_t total = (gbytes + 255) & ~(size_t)255;
         if (send_expect) total += (ebytes + 255) & ~(size_t)255;
         if (send_lgt) total += (lbytes + 255) & ~(size_t)255;
         if ((e = stage.begin(total)) != hipSuccess) return e;
         if ((e = stage.copy(geom.ptr, gs.data(), gbytes, st)) != hipSuccess) return e;
-        if ((e = stage.copy(flag.ptr, &zero, sizeof(zero), st)) != hipSuccess) return e;
         if (send_expect && (e = stage.copy(expect.ptr, want.data(), ebytes, st)) != hipSuccess)
         {
             return e;
@@ -475,10 +482,20 @@ struct DevTables
         }
         if ((e = stage.end(st)) != hipSuccess) return e;
         if (send_expect) expect_build = build_on_dev;
+        t.spawns = 0;
+        for (const qr_geom &g : gs)
+        {
+            if (g.tag != RT_TAG_ARRAY && (qr_side_spawns(g.props[0]) || qr_side_spawns(g.props[1])))
+            {
+                t.spawns = 1;
+            }
+        }
+        /* (the last update's kernels are done: it waited for them) */
+        *flag_host = 0u;
         e = qr_update_records((const qr_geom *)geom.ptr, h.n_surf, (const qr_clip *)clp.ptr,
                               (qr_surface *)srf.ptr, (qr_dev_surf *)hot.ptr,
                               (qr_material *)mat.ptr, (qr_refit_elem *)refit_in.ptr,
-                              (const int32_t *)expect.ptr, (uint32_t *)flag.ptr, st);
+                              (const int32_t *)expect.ptr, flag_host, st);
         if (e != hipSuccess) return e;
         e = qr_refit_programs((qr_dev_step *)step.ptr, dev_n_step,
                               any ? (qr_dev_step *)step_any.ptr : nullptr, any ? dev_n_any : 0,
@@ -486,11 +503,6 @@ struct DevTables
                               (const qr_surface *)srf.ptr, t.cull_ref,
                               (float *)refit_box.ptr, st);
         if (e != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(flag_host, flag.ptr, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                st)) != hipSuccess)
-        {
-            return e;
-        }
         if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
         /* the device now holds records, materials and boxes no host copy has */
         for (int i : {0, 1, 2, 3}) sent[i].clear();

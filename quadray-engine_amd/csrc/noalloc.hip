@@ -229,6 +229,7 @@ int qrhip_render_tables_noalloc(qrhip_dev *dev, const qr_scene_tables *tab,
     t.n_clip = tab->n_clip;
     t.n_elem = tab->n_elem;
     t.n_texel = tab->n_texel;
+    t.spawns = 1;
 
     qr_frame_desc d = *fd;
     d.x_row = fd->x_res;

@@ -355,9 +355,11 @@ void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
                 {
                     by_time = (int)std::max(1.0, (budget_ms - used_ms - fixed) / pass_ms);
                 }
-                else
+                else if (cap == ~0ull)
                 {
-                    by_time = 1;
+                    /* whole frames: as many passes as a run of 2^24 samples */
+                    by_time = (int)std::max<uint64_t>(1, std::min<uint64_t>(
+                        (uint64_t)left, (1ull << 24) / std::max<uint64_t>(1, ch.cost)));
                 }
                 if (cap != ~0ull)
                 {

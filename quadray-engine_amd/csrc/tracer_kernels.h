@@ -252,7 +252,15 @@ typedef struct qr_device_tables
     qr_dev_step *steps_any;     /* any-hit culling program (n_step_any + 1) */
     int32_t      n_surf, n_mat, n_lgt, n_clip, n_elem, n_texel, n_step, n_step_any;
     float        cull_ref[4];   /* reference point of the world boxes */
+    int32_t      spawns;        /* some surface reflects or transmits: a frame of
+                                   a scene where none does has no secondary
+                                   rays at any depth */
 } qr_device_tables;
+/* does a hit on a side with these properties have children (trrf_setup) */
+static inline int qr_side_spawns(uint32_t props)
+{
+    return (props & QR_PROP_REFLECT) != 0 || (props & QR_PROP_OPAQUE) == 0;
+}
 
 /* hot[i] from srf[i] for every record, on the device */
 hipError_t qr_dev_surfaces(const qr_surface *srf, int n, qr_dev_surf *hot, hipStream_t stream);

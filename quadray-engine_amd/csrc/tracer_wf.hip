@@ -152,6 +152,8 @@ struct Batch
                                        shadow walks and shading (-1: none) */
     int32_t            rpt;         /* blocks of WG entries per virtual
                                        workgroup (rays per thread) */
+    uint32_t          *cnt_host;    /* the resolve's copy of the counter blocks,
+                                       in the host's page-locked memory */
 };
 
 /* plan kinds */
@@ -920,6 +922,12 @@ __global__ void __launch_bounds__(WG) k_resolve(Batch b)
 {
     const int rpt = R != 0 ? R : b.rpt;    /* rays per thread; R = 1: every level dense */
     const uint32_t total = launch_total(b, PLAN_LEVEL);
+    /* the counters, final by now, to the host (a copy behind the launch
+     * would be one more operation to wait for) */
+    for (int f = blockIdx.x; f < b.nfr; f += gridDim.x)
+    {
+        if (threadIdx.x < CNT_N) b.cnt_host[f * CNT_N + threadIdx.x] = b.fr[f].cnt[threadIdx.x];
+    }
     for (uint32_t vb = blockIdx.x; vb < total; vb += gridDim.x)
     {
         const int f = launch_frame(b, vb);
@@ -1237,6 +1245,14 @@ static hipError_t frame_reserve(qr_wf_state *s, const qr_device_tables *t, uint6
     return hipSuccess;
 }
 
+/* camera samples up to which a single frame's level-0 shadow walks and level-1
+ * nearest walks share one stage kernel instead of running side by side on
+ * two streams: a 64x64 frame 0.222 -> 0.207 ms, 640x360 0.391 -> 0.383 (the
+ * second stream's fork and join cost about 10 us), 1281x719 2X the same;
+ * larger frames win it back with each kernel's own register budget (1080p 4X
+ * 1.756 ms on two streams, 1.866 in one launch) */
+constexpr uint64_t SMALL_SAMPLES = 1u << 20;
+
 /* one launch after the camera samples' nearest walks: its levels of nearest
  * walks, shadow walks and shading (-1: none) */
 struct Stage
@@ -1248,19 +1264,34 @@ struct Stage
  * level's shadow walks follow its nearest walks and precede its shading
  * (level 0's shading is part of the resolve).  The camera samples' shadow
  * walks and the nearest walks of level 1 fill the chip by themselves and
- * run alone; from then on stage j runs the nearest walks of level j, the
+ * run alone (of a small frame, they share a launch); from then on stage j runs the nearest walks of level j, the
  * shadow walks of level j-1 and the shading of level j-2 side by side */
-static std::vector<Stage> stage_list(int levels)
+static std::vector<Stage> stage_list(int levels, bool small)
 {
     std::vector<Stage> st;
     auto lv = [&](int L) { return L >= 0 && L < levels ? L : -1; };
-    st.push_back({-1, 0, -1});
-    st.push_back({lv(1), -1, -1});
+    if (small)
+    {
+        st.push_back({lv(1), 0, -1});
+    }
+    else
+    {
+        st.push_back({-1, 0, -1});
+        st.push_back({lv(1), -1, -1});
+    }
     for (int j = 2; j <= levels + 1; j++) st.push_back({lv(j), lv(j - 1), j >= 3 ? lv(j - 2) : -1});
     st.erase(std::remove_if(st.begin(), st.end(),
                             [](const Stage &x) { return x.wl < 0 && x.sl < 0 && x.fl < 0; }),
              st.end());
     return st;
+}
+
+/* tree levels of a frame: its depth and the camera samples, or the camera
+ * samples alone where no surface has children (an 800x480 frame of the plain
+ * scene then takes 4 launches instead of 10, with its copies 0.159 -> 0.127 ms) */
+static int frame_levels(const qr_wf_item &it)
+{
+    return it.t->spawns != 0 ? it.fd->depth + 1 : 1;
 }
 
 hipError_t qr_wf_batch_launch(qr_wf_batch *b, const qr_wf_item *items, int n,
@@ -1277,7 +1308,7 @@ hipError_t qr_wf_batch_launch(qr_wf_batch *b, const qr_wf_item *items, int n,
         {
             return hipErrorInvalidValue;
         }
-        levels = std::max(levels, fd->depth + 1);
+        levels = std::max(levels, frame_levels(items[k]));
     }
 
     /* counters and plans */
@@ -1321,7 +1352,7 @@ hipError_t qr_wf_batch_launch(qr_wf_batch *b, const qr_wf_item *items, int n,
         if (tile0 + ntiles > all) return hipErrorInvalidValue;
         const uint64_t n0 = ntiles * TILE_PX * ns;
         if (n0 > 0x7fffff00ull) return hipErrorInvalidValue;
-        const int lv = fd->depth + 1;
+        const int lv = frame_levels(it);
         if ((e = frame_reserve(it.s, it.t, n0, lv)) != hipSuccess) return e;
 
         Frame &a = fr[k];
@@ -1389,11 +1420,16 @@ hipError_t qr_wf_batch_launch(qr_wf_batch *b, const qr_wf_item *items, int n,
     bt.level = 0;
     bt.wl = bt.sl = bt.fl = -1;
     bt.rpt = b->rpt;
+    bt.cnt_host = b->cnt_host;
     /* the persistent grid, but no more workgroups than the camera samples
      * fill: a small batch (a chunk of a served step, a thumbnail) does not
      * pay for thousands of empty workgroups per launch */
-    uint64_t wg0 = 0;
-    for (const Frame &a : fr) wg0 += ((uint64_t)a.n0 + WG - 1) / WG;
+    uint64_t wg0 = 0, samples = 0;
+    for (const Frame &a : fr)
+    {
+        wg0 += ((uint64_t)a.n0 + WG - 1) / WG;
+        samples += a.n0;
+    }
     const unsigned gfit = (unsigned)std::min<uint64_t>(
         (uint64_t)b->grid, std::max<uint64_t>(wg0, (uint64_t)b->cus));
     const dim3 g(gfit), w(WG);
@@ -1414,14 +1450,14 @@ hipError_t qr_wf_batch_launch(qr_wf_batch *b, const qr_wf_item *items, int n,
     };
     hipLaunchKernelGGL(k_reset, dim3((unsigned)std::min(n, 1024)), w, 0, stream, bt);
     hipLaunchKernelGGL(one ? k_walk0<1> : k_walk0<0>, g, w, 0, stream, plan(PLAN_LEVEL, 0));
-    const std::vector<Stage> stages = stage_list(levels);
+    const std::vector<Stage> stages = stage_list(levels, !planned && samples <= SMALL_SAMPLES);
     /* Only the resolve reads the camera samples' shadow walks (stage 0),
      * whose queue set, visibility masks and counters no other stage
      * touches: outside graph capture they run on a second stream beside
      * all the deeper stages and folds, each kernel with its own register
      * budget, and the resolve waits for them. */
     hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
-    const bool overlap = !stages.empty() && stages[0].sl == 0 && stages[0].wl < 0 &&
+    const bool overlap = stages.size() > 1 && stages[0].sl == 0 && stages[0].wl < 0 &&
                          stages[0].fl < 0 &&
                          hipStreamIsCapturing(stream, &cap) == hipSuccess &&
                          cap == hipStreamCaptureStatusNone;
@@ -1483,9 +1519,7 @@ hipError_t qr_wf_batch_launch(qr_wf_batch *b, const qr_wf_item *items, int n,
     Batch pr = bt;
     if (planned) pr.plan = (const QC uint32_t *)plan_of(PLAN_LEVEL, 0);
     hipLaunchKernelGGL(one ? k_resolve<1> : k_resolve<0>, g, w, 0, stream, pr);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    return hipMemcpyAsync(b->cnt_host, b->cnt.ptr, sizeof(uint32_t) * CNT_N * (size_t)n,
-                          hipMemcpyDeviceToHost, stream);
+    return hipGetLastError();
 }
 
 int qr_wf_batch_check(qr_wf_batch *b, const qr_wf_item *items, int n)

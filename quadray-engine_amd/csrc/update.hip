@@ -120,8 +120,9 @@ __global__ void __launch_bounds__(RF_WG) k_boxes(qr_dev_step *prog0, int n0, qr_
 
 /* every record of the table: one work-item each.  expect holds, per
  * element, the world and local box flags the programs were built for; an
- * element whose flags differ sets *mismatch (the programs' structure no
- * longer fits: the host rebuilds them) */
+ * element whose flags differ sets *mismatch, in the host's page-locked
+ * memory (the programs' structure no longer fits: the host rebuilds them; a
+ * flag in device memory cost two copies an update, 15 us of a small frame) */
 __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
                                                  const qr_clip *clips, qr_surface *srf,
                                                  qr_dev_surf *hot, qr_material *mat,
@@ -142,7 +143,7 @@ __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
             qr_refit_elem z;
             memset(&z, 0, sizeof(z));
             refit_in[g.elem] = z;
-            if (expect[2 * g.elem] != 0 || expect[2 * g.elem + 1] != 0) atomicOr(mismatch, 1u);
+            if (expect[2 * g.elem] != 0 || expect[2 * g.elem + 1] != 0) *mismatch = 1u;
         }
         return;
     }
@@ -174,7 +175,7 @@ __global__ void __launch_bounds__(64) k_records(const qr_geom *geoms, int n_rec,
         refit_in[g.elem] = e;
         if (expect[2 * g.elem] != e.world || expect[2 * g.elem + 1] != e.local)
         {
-            atomicOr(mismatch, 1u);
+            *mismatch = 1u;
         }
     }
 }

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import qrhip
-from helpers import oracle_rows
+from helpers import HostScene, oracle_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -322,3 +322,25 @@ def test_batch_download_parts(device, sizes):
                 s.destroy()
                 w.close()
             assert np.array_equal(f, want), f"frame {x}x{y} pad {pad}"
+
+
+def test_batch_with_and_without_secondary_rays(device):
+    """Scenes with no reflecting or transparent surface (no levels below the
+    camera samples at any depth) beside scenes with deep trees, in one batch
+    and alone, against the oracle."""
+    scenes = [(1, 6), (6, 4), (1, 9)]
+    reqs = [(0, 65, 33, 2, 4), (1, 48, 31, 0, 5), (2, 17, 9, 1, 14), (0, 8, 8, 0, 0)]
+    bc = BatchCase(device, scenes, reqs)
+    try:
+        got = bc.batch.render(qrhip.BATCH_DIRECT)
+    finally:
+        bc.close()
+    for key, frame in zip(bc.keys, got):
+        config, seed, x, y, fsaa, depth = key
+        hs = HostScene(config, seed, x, y, fsaa, depth)
+        try:
+            want = hs.oracle()[0]
+        finally:
+            hs.close()
+        assert np.array_equal(frame, want), f"batched frame {key}"
+        assert np.array_equal(alone(device, *key), want), f"frame {key} alone"
