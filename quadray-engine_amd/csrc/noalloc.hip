@@ -229,7 +229,16 @@ int qrhip_render_tables_noalloc(qrhip_dev *dev, const qr_scene_tables *tab,
     t.n_clip = tab->n_clip;
     t.n_elem = tab->n_elem;
     t.n_texel = tab->n_texel;
-    t.spawns = 1;
+    t.spawns = 0;
+    for (int i = 0; i < tab->n_surf; i++)
+    {
+        const qr_surface &s = tab->surfaces[i];
+        if (s.solver != QR_SOLVE_NONE && (qr_side_spawns(s.props[0]) || qr_side_spawns(s.props[1])))
+        {
+            t.spawns = 1;
+            break;
+        }
+    }
 
     qr_frame_desc d = *fd;
     d.x_row = fd->x_res;

@@ -1,14 +1,30 @@
 /*
  * tracer.hip -- one-kernel Whitted tracer for MI355X (gfx950).
  *
- * One work-item per pixel, looping over its anti-aliasing sub-samples; the
- * whole reflection / refraction tree of a sample is traced inside the
- * kernel.  QuadRay's recursive context stack (shadow, refraction and
- * reflection rays re-entering the list walk, core/tracer/tracer.cpp
- * 4046-4077, 4770-4862, 5160-5277) becomes an explicit per-lane stack of
- * pending tree nodes; colours are accumulated bottom-up in QuadRay's order.
+ * 1 to 16 work-items per camera sample (the fewer samples, the more); the
+ * whole reflection / refraction tree of a sample is traced inside the kernel.
+ * QuadRay's recursive context stack (shadow, refraction and reflection rays
+ * re-entering the list walk, core/tracer/tracer.cpp 4046-4077, 4770-4862,
+ * 5160-5277) becomes an explicit per-lane stack of pending tree nodes;
+ * colours are accumulated bottom-up in QuadRay's order.
  * The level-by-level pipeline (tracer_wf.hip) is the default path; this
- * kernel serves scenes beyond that pipeline's light-mask limit.
+ * kernel serves scenes beyond that pipeline's light-mask limit, and callers
+ * that cannot allocate.
+ *
+ * Its time is that of its longest waves, whose lanes' trees are walked node
+ * by node while the rest of the chip has run dry (vector issue was 4% busy
+ * over a 640x360 frame of glass and mirrors at 2 samples).  So a lane takes
+ * one sample, not a pixel's one after another, and where the frame leaves the
+ * chip idle a wave holds fewer samples (its walks test only surfaces that
+ * some lane of it needs, and the union of 4 samples' trees is shorter than
+ * that of 64), SPLIT lanes each, which follow the same rays and test that
+ * many lights' shadow rays at once: a node in a scene of four lights costs
+ * two walks instead of five.
+ *
+ * Times, one pixel per lane before -> now: 640x360 at 2 samples, depth 4:
+ * 2.55 -> 0.61 ms; 641x359 at 4, depth 8: 102 -> 11.0; 1281x719 at 2:
+ * 9.6 -> 3.6; 64x64: 1.12 -> 0.31; 1920x1080 at 4: 5.3 -> 1.8; 800x480
+ * without secondary rays: 0.020 -> 0.019.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -36,9 +52,12 @@ __device__ __forceinline__ Ray child(const Node &nd, int which)
 /* one camera sample through the whole Whitted tree: a node waits on the
  * stack for its refraction child, then its reflection child, and folds each
  * result into its colour as QuadRay's TR_mix / RF_mix do */
+template <int SPLIT>
 __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
                            int32_t *hit_id)
 {
+    const int sub = (int)(threadIdx.x & (SPLIT - 1));
+    const int group = __lane_id() & ~(SPLIT - 1);
     Node stk[MAX_STACK];
     int sp = 0;
     V3 ret = {0.0f, 0.0f, 0.0f};
@@ -60,10 +79,40 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
             hit_info(sc, ray, h);
             const V3 nrm = normal_at(sc, h);
             Node &nd = stk[sp];
-            shade(sc, fd, ray, h, nrm, nd, [&](int, const Ray &sr) {
-                Hit sh;
-                return walk<true>(sc, sr, sh);
-            });
+            V3 tex;
+            bool lit;
+            V3 col = shade_base(sc, fd, h, tex, lit);
+            for (int l0 = 0; lit && l0 < sc.n_lgt; l0 += SPLIT)
+            {
+                /* this lane's light of the next four, then all four added in
+                 * their order */
+                const int li = l0 + sub;
+                Ray sr;
+                bool vis = li < sc.n_lgt && 0.0f < light_vec(sc.lgt[li], h.hit, nrm, sr.dir);
+                if (vis)
+                {
+                    sr.org = h.hit;
+                    sr.t_min = 0.0f;
+                    sr.t_max = sc.lgt[li].t_max;
+                    sr.flags = h.side | FLAG_SHAD;
+                    sr.origin = h.srf;
+                    sr.oloc = h.loc;
+                    sr.depth = 0;
+                    Hit sh;
+                    vis = !walk<true>(sc, sr, sh);
+                }
+                const uint32_t four = (uint32_t)(lanes(vis) >> group);
+                for (int k = 0; k < SPLIT && l0 + k < sc.n_lgt; k++)
+                {
+                    if (!((four >> k) & 1u)) continue;
+                    const QC qr_light &l = sc.lgt[l0 + k];
+                    V3 L;
+                    const float dot = light_vec(l, h.hit, nrm, L);
+                    shade_light(sc, l, ray.dir, h, nrm, tex, L, dot, col);
+                }
+            }
+            nd.col = col;
+            node_children(sc, ray, h, nrm, nd);
             if (nd.todo & 1)
             {
                 nd.todo |= 4;
@@ -119,17 +168,40 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
     }
 }
 
+constexpr int log2i(int n) { return n < 2 ? 0 : 1 + log2i(n / 2); }
+
+/* a wave's tile of pixels: its 64 / SPLIT samples, ns to a pixel, as near to
+ * square as powers of two allow (wider before higher) */
+template <int SPLIT>
+__host__ __device__ constexpr int tile_w(int ns)
+{
+    return 1 << ((log2i(64 / SPLIT / ns) + 1) / 2);
+}
+template <int SPLIT>
+__host__ __device__ constexpr int tile_h(int ns)
+{
+    return 1 << (log2i(64 / SPLIT / ns) / 2);
+}
+
+/* four waves per workgroup, their tiles side by side; a pixel's samples in neighbouring
+ * groups of SPLIT lanes */
+template <int SPLIT>
 __global__ void __launch_bounds__(256)
-whitted_kernel(Scene sc, qr_frame_desc fd, uint32_t *__restrict__ frame,
+whitted_kernel(Scene sc, qr_frame_desc fd, int ns, uint32_t *__restrict__ frame,
                int32_t *__restrict__ ids)
 {
-    const int x = blockIdx.x * 16 + (threadIdx.x & 15);
-    const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (x >= fd.x_res || y >= fd.y_res) return;
+    const int tw = ns == 1 ? tile_w<SPLIT>(1) : ns == 2 ? tile_w<SPLIT>(2) : tile_w<SPLIT>(4);
+    const int th = ns == 1 ? tile_h<SPLIT>(1) : ns == 2 ? tile_h<SPLIT>(2) : tile_h<SPLIT>(4);
+    const int wv = threadIdx.x / 64;
+    const int s = (threadIdx.x & 63) / SPLIT;
+    const int p = s / ns, k = s - p * ns;
+    const int x = (blockIdx.x * 4 + wv) * tw + p % tw;
+    const int y = (blockIdx.z * gridDim.y + blockIdx.y) * th + p / tw;
+    const bool in = x < fd.x_res && y < fd.y_res;
+    const bool first = (threadIdx.x & (SPLIT - 1)) == 0;
 
-    const int ns = fd.fsaa == 2 ? 4 : fd.fsaa == 1 ? 2 : 1;
-    V3 acc[4];
-    for (int k = 0; k < ns; k++)
+    V3 c = V3{0.0f, 0.0f, 0.0f};
+    if (in)
     {
         int sk = k;
         if (fd.fsaa == 1 && (x & 1)) sk = k + 2;
@@ -153,49 +225,28 @@ whitted_kernel(Scene sc, qr_frame_desc fd, uint32_t *__restrict__ frame,
         r.oloc = V3{0.0f, 0.0f, 0.0f};
         r.depth = fd.depth;
         int32_t id;
-        V3 c = trace_sample(sc, fd, r, &id);
-        acc[k].x = c.x < 1.0f ? c.x : 1.0f;
-        acc[k].y = c.y < 1.0f ? c.y : 1.0f;
-        acc[k].z = c.z < 1.0f ? c.z : 1.0f;
-        if (ids != nullptr)
+        c = trace_sample<SPLIT>(sc, fd, r, &id);
+        c.x = c.x < 1.0f ? c.x : 1.0f;
+        c.y = c.y < 1.0f ? c.y : 1.0f;
+        c.z = c.z < 1.0f ? c.z : 1.0f;
+        if (ids != nullptr && first)
         {
             ids[((size_t)y * fd.x_res + x) * ns + k] = id;
         }
     }
+    const uint32_t px = resolve_lanes<SPLIT>(fd, ns, c);
+    if (in && first && k == 0) frame[(ptrdiff_t)y * fd.x_row + x] = px;
+}
 
-    V3 c;
-    if (ns == 1)
-    {
-        c = acc[0];
-    }
-    else if (ns == 2)
-    {
-        c.x = acc[0].x * 0.5f + acc[1].x * 0.5f;
-        c.y = acc[0].y * 0.5f + acc[1].y * 0.5f;
-        c.z = acc[0].z * 0.5f + acc[1].z * 0.5f;
-    }
-    else
-    {
-        float p0, p1;
-        p0 = acc[0].x * 0.5f + acc[1].x * 0.5f; p1 = acc[2].x * 0.5f + acc[3].x * 0.5f;
-        c.x = p0 * 0.5f + p1 * 0.5f;
-        p0 = acc[0].y * 0.5f + acc[1].y * 0.5f; p1 = acc[2].y * 0.5f + acc[3].y * 0.5f;
-        c.y = p0 * 0.5f + p1 * 0.5f;
-        p0 = acc[0].z * 0.5f + acc[1].z * 0.5f; p1 = acc[2].z * 0.5f + acc[3].z * 0.5f;
-        c.z = p0 * 0.5f + p1 * 0.5f;
-    }
-
-    float v[3] = {c.x, c.y, c.z};
-    uint32_t px = 0;
-    #pragma unroll
-    for (int a = 0; a < 3; a++)
-    {
-        float f = v[a];
-        if (fd.gamma & QR_PROP_GAMMA) f = sqrtf(f);
-        f = f * 255.0f;
-        px |= ((uint32_t)cvt_rne(f) & 0xFFu) << (16 - 8 * a);
-    }
-    frame[(ptrdiff_t)y * fd.x_row + x] = px;
+template <int SPLIT>
+void launch(const Scene &sc, const qr_frame_desc &fd, int ns, uint32_t *frame, int32_t *ids,
+            hipStream_t stream)
+{
+    const int tw = 4 * tile_w<SPLIT>(ns), th = tile_h<SPLIT>(ns);
+    const unsigned nx = (unsigned)((fd.x_res - 1) / tw + 1), ny = (unsigned)((fd.y_res - 1) / th + 1);
+    const unsigned gy = ny < 65535u ? ny : 65535u;
+    hipLaunchKernelGGL(whitted_kernel<SPLIT>, dim3(nx, gy, (ny + gy - 1) / gy), dim3(256), 0, stream,
+                       sc, fd, ns, frame, ids);
 }
 
 } /* namespace */
@@ -208,8 +259,19 @@ hipError_t qr_launch_whitted(const qr_device_tables *t, const qr_frame_desc *fd,
     {
         return hipErrorInvalidValue;
     }
-    dim3 grid((fd->x_res + 15) / 16, (fd->y_res + 15) / 16);
-    hipLaunchKernelGGL(whitted_kernel, grid, dim3(256), 0, stream, sc, *fd,
-                       frame, ids);
+    const int ns = fd->fsaa == 2 ? 4 : fd->fsaa == 1 ? 2 : 1;
+    /* lanes per sample, by how many samples there are to fill the chip (a
+     * frame without secondary rays, whose waves all take about as long, fills
+     * it with a sixteenth).  ms at 1, 2, 4 and 16 lanes: 320x180 1.43 0.89
+     * 0.55 0.37; 640x360 at 2 samples 1.22 0.83 0.61 0.89; 1920x1080 1.32 1.09
+     * 0.96 2.68; at 2 samples 1.49 1.30 1.51 5.41; at 4 1.80 1.88 2.99 9.75;
+     * without secondary rays, 64x64 0.148 0.092 0.060 0.048; 640x360 at 2
+     * 0.089 0.089 0.125 0.431 (8 lanes lie between 4 and 16) */
+    const bool tree = t->spawns && fd->depth > 0;
+    const uint64_t n = (uint64_t)fd->x_res * (uint64_t)fd->y_res * (uint64_t)ns * (tree ? 1u : 16u);
+    if (n <= (1u << 18)) launch<16>(sc, *fd, ns, frame, ids, stream);
+    else if (n <= (1u << 21)) launch<4>(sc, *fd, ns, frame, ids, stream);
+    else if (n <= (1u << 22)) launch<2>(sc, *fd, ns, frame, ids, stream);
+    else launch<1>(sc, *fd, ns, frame, ids, stream);
     return hipGetLastError();
 }

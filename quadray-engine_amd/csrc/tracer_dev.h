@@ -1359,13 +1359,14 @@ __device__ __forceinline__ uint32_t resolve_pack(const qr_frame_desc &fd, int ns
     return pack_argb(fd, c);
 }
 
-/* the same resolve of a pixel's samples held by ns neighbouring lanes
- * (sample k in lane k of an aligned group): halve, then add the partner
- * lane's value per pass; every lane of the wave calls it with the same ns,
- * and each lane of the group gets the pixel */
+/* the same resolve of a pixel's samples held by ns neighbouring groups of
+ * "span" lanes (sample k in group k of an aligned run of groups): halve,
+ * then add the partner's value per pass; every lane of the wave calls it with
+ * the same ns, and each lane of the groups gets the pixel */
+template <int span = 1>
 __device__ __forceinline__ uint32_t resolve_lanes(const qr_frame_desc &fd, int ns, V3 c)
 {
-    for (int d = 1; d < ns; d <<= 1)
+    for (int d = span; d < ns * span; d <<= 1)
     {
         const V3 h = V3{c.x * 0.5f, c.y * 0.5f, c.z * 0.5f};
         c.x = h.x + __shfl_xor(h.x, d);
@@ -1388,115 +1389,121 @@ struct Node
     int   todo;         /* bit 0: refraction pending, bit 1: reflection */
 };
 
-/* local shading of a hit (MT, LT): its colour; occluded(light, shadow ray)
- * answers the hard-shadow test of one light */
-template <class Occluded>
-__device__ V3 shade_color(const Scene &sc, const qr_frame_desc &fd, const Ray &r,
-                          const Hit &h, const V3 &nrm, Occluded occluded)
+/* colour of a hit without its lights (MT): a LIGHT material's own colour
+ * ("lit" false), or the ambient part, with the texel the lights use */
+__device__ __forceinline__ V3 shade_base(const Scene &sc, const qr_frame_desc &fd, const Hit &h,
+                                         V3 &tex, bool &lit)
 {
     const QC qr_surface &s = sc.srf[h.srf];
     const uint32_t props = s.props[h.side];
     const QC qr_material &m = sc.mat[s.mat[h.side]];
-
-    const V3 tex = texel_color(sc, m, props, h);
-
+    tex = texel_color(sc, m, props, h);
+    lit = !(props & QR_PROP_LIGHT);
+    if (!lit) return tex;
     V3 col;
-    if (props & QR_PROP_LIGHT)
+    col.x = tex.x * fd.amb[0];
+    col.y = tex.y * fd.amb[1];
+    col.z = tex.z * fd.amb[2];
+    float f = 1.0f - m.c_trn;
+    f = f - m.c_rfl;
+    if (!(0.0f <= f)) f = 0.0f;
+    col.x = col.x * f;
+    col.y = col.y * f;
+    col.z = col.z * f;
+    return col;
+}
+
+/* a visible light's part of a hit's colour added to it (LT): L the vector to
+ * the light, dot its product with the normal, rdir the ray's direction */
+__device__ __forceinline__ void shade_light(const Scene &sc, const QC qr_light &l, const V3 &rdir,
+                                            const Hit &h, const V3 &nrm, const V3 &tex, const V3 &L,
+                                            float dot, V3 &col)
+{
+    const QC qr_surface &s = sc.srf[h.srf];
+    const uint32_t props = s.props[h.side];
+    const QC qr_material &m = sc.mat[s.mat[h.side]];
+    float r2 = L.x * L.x + L.y * L.y;
+    r2 = r2 + L.z * L.z;
+
+    float dff = 0.0f;
+    if (props & QR_PROP_DIFFUSE)
     {
-        col = tex;
+        float ir = rsq(r2);
+        float r1 = ir * r2;
+        float at = r2 * l.a_qdr;
+        float lr = r1 * l.a_lnr;
+        at = at + l.a_cnt;
+        at = at + lr;
+        float ia = rsq(at);
+        dff = dot * ia;
+        dff = dff * ir;
+        dff = dff * m.l_dff;
+    }
+
+    bool plain_spc = false;
+    float spc = 0.0f;
+    if (props & QR_PROP_SPECULAR)
+    {
+        V3 R;
+        float v = dot * nrm.x;
+        R.x = L.x - v; R.x = R.x - v;
+        v = dot * nrm.y;
+        R.y = L.y - v; R.y = R.y - v;
+        v = dot * nrm.z;
+        R.z = L.z - v; R.z = R.z - v;
+        float rr2 = rdir.z * rdir.z;
+        rr2 = rr2 + rdir.x * rdir.x;
+        rr2 = rr2 + rdir.y * rdir.y;
+        float sn = R.x * rdir.x + R.y * rdir.y;
+        sn = sn + R.z * rdir.z;
+        if (0.0f < sn)
+        {
+            sn = sn * rsq(rr2);
+            sn = sn * rsq(r2);
+            spc = spec_pow(sn, m.l_pow);
+            spc = spc * m.l_spc;
+            if (props & QR_PROP_METAL) dff = dff + spc;
+            else plain_spc = true;
+        }
+    }
+
+    V3 lc;
+    if (plain_spc)
+    {
+        float v;
+        v = tex.x * dff; v = v * l.col[0]; lc.x = v + l.col[0] * spc;
+        v = tex.y * dff; v = v * l.col[1]; lc.y = v + l.col[1] * spc;
+        v = tex.z * dff; v = v * l.col[2]; lc.z = v + l.col[2] * spc;
     }
     else
     {
-        col.x = tex.x * fd.amb[0];
-        col.y = tex.y * fd.amb[1];
-        col.z = tex.z * fd.amb[2];
-        float f = 1.0f - m.c_trn;
-        f = f - m.c_rfl;
-        if (!(0.0f <= f)) f = 0.0f;
-        col.x = col.x * f;
-        col.y = col.y * f;
-        col.z = col.z * f;
+        lc.x = (tex.x * l.col[0]) * dff;
+        lc.y = (tex.y * l.col[1]) * dff;
+        lc.z = (tex.z * l.col[2]) * dff;
+    }
+    col.x = lc.x + col.x;
+    col.y = lc.y + col.y;
+    col.z = lc.z + col.z;
+}
 
+/* local shading of a hit (MT, LT): its colour; visible(light) answers the
+ * hard-shadow test of one light facing it */
+template <class Visible>
+__device__ V3 shade_color(const Scene &sc, const qr_frame_desc &fd, const V3 &rdir, const Hit &h,
+                          const V3 &nrm, Visible visible)
+{
+    V3 tex;
+    bool lit;
+    V3 col = shade_base(sc, fd, h, tex, lit);
+    if (lit)
+    {
         for (int li = 0; li < sc.n_lgt; li++)
         {
             const QC qr_light &l = sc.lgt[li];
             V3 L;
             const float dot = light_vec(l, h.hit, nrm, L);
-            if (!(0.0f < dot)) continue;
-
-            Ray sr;
-            sr.org = h.hit;
-            sr.dir = L;
-            sr.t_min = 0.0f;
-            sr.t_max = l.t_max;
-            sr.flags = h.side | FLAG_SHAD;
-            sr.origin = h.srf;
-            sr.oloc = h.loc;
-            sr.depth = r.depth - 1;
-            if (occluded(li, sr)) continue;
-
-            float r2 = L.x * L.x + L.y * L.y;
-            r2 = r2 + L.z * L.z;
-
-            float dff = 0.0f;
-            if (props & QR_PROP_DIFFUSE)
-            {
-                float ir = rsq(r2);
-                float r1 = ir * r2;
-                float at = r2 * l.a_qdr;
-                float lr = r1 * l.a_lnr;
-                at = at + l.a_cnt;
-                at = at + lr;
-                float ia = rsq(at);
-                dff = dot * ia;
-                dff = dff * ir;
-                dff = dff * m.l_dff;
-            }
-
-            bool plain_spc = false;
-            float spc = 0.0f;
-            if (props & QR_PROP_SPECULAR)
-            {
-                V3 R;
-                float v = dot * nrm.x;
-                R.x = L.x - v; R.x = R.x - v;
-                v = dot * nrm.y;
-                R.y = L.y - v; R.y = R.y - v;
-                v = dot * nrm.z;
-                R.z = L.z - v; R.z = R.z - v;
-                float rr2 = r.dir.z * r.dir.z;
-                rr2 = rr2 + r.dir.x * r.dir.x;
-                rr2 = rr2 + r.dir.y * r.dir.y;
-                float sn = R.x * r.dir.x + R.y * r.dir.y;
-                sn = sn + R.z * r.dir.z;
-                if (0.0f < sn)
-                {
-                    sn = sn * rsq(rr2);
-                    sn = sn * rsq(r2);
-                    spc = spec_pow(sn, m.l_pow);
-                    spc = spc * m.l_spc;
-                    if (props & QR_PROP_METAL) dff = dff + spc;
-                    else plain_spc = true;
-                }
-            }
-
-            V3 lc;
-            if (plain_spc)
-            {
-                float v;
-                v = tex.x * dff; v = v * l.col[0]; lc.x = v + l.col[0] * spc;
-                v = tex.y * dff; v = v * l.col[1]; lc.y = v + l.col[1] * spc;
-                v = tex.z * dff; v = v * l.col[2]; lc.z = v + l.col[2] * spc;
-            }
-            else
-            {
-                lc.x = (tex.x * l.col[0]) * dff;
-                lc.y = (tex.y * l.col[1]) * dff;
-                lc.z = (tex.z * l.col[2]) * dff;
-            }
-            col.x = lc.x + col.x;
-            col.y = lc.y + col.y;
-            col.z = lc.z + col.z;
+            if (!(0.0f < dot) || !visible(li)) continue;
+            shade_light(sc, l, rdir, h, nrm, tex, L, dot, col);
         }
     }
     return col;
@@ -1524,15 +1531,6 @@ __device__ __forceinline__ void node_children(const Scene &sc, const Ray &r, con
     nd.c_trn = t.c_trn;
     nd.c_rfl = t.c_rfl;
     if (r.depth == 0) nd.todo = 0;
-}
-
-/* local shading of a hit and set-up of its children (MT, LT, TR, RF) */
-template <class Occluded>
-__device__ void shade(const Scene &sc, const qr_frame_desc &fd, const Ray &r,
-                      const Hit &h, const V3 &nrm, Node &nd, Occluded occluded)
-{
-    nd.col = shade_color(sc, fd, r, h, nrm, occluded);
-    node_children(sc, r, h, nrm, nd);
 }
 
 } /* namespace */

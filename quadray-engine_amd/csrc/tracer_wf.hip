@@ -689,9 +689,9 @@ __device__ __forceinline__ V3 hit_color(const QC Frame &a, const Level &cur, int
         const V3 nrm = V3{nc.x, nc.y, nc.z};
         const uint32_t vis = cur.vis[i];
         const qr_frame_desc fd = ldc(a.fd);
-        col = shade_color(sc, fd, r, h, nrm, [&](int li, const Ray &) {
+        col = shade_color(sc, fd, r.dir, h, nrm, [&](int li) {
             const int bit = sc.n_lgt <= VIS_BYTE_LIGHTS ? 8 * li : li;
-            return ((vis >> bit) & 1u) == 0u;
+            return ((vis >> bit) & 1u) != 0u;
         });
     }
     return col;

@@ -340,3 +340,29 @@ def test_gpu_root_forms(path_dev, config, seed, d_eps, zero):
     got, ids = path_dev.render_tables(t.ptr, t.fd, want_ids=True)
     assert_frame_exact(got, want, f"config {config} d_eps {d_eps} zero {zero}")
     assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
+
+
+@pytest.mark.parametrize("config,x,y,fsaa,depth", [
+    # 16 lanes to a sample: the smallest frame, ragged edges of every tile
+    # shape, the largest number of samples; then 4, 2 and 1 lanes
+    (2, 1, 1, 0, 4), (4, 37, 23, 1, 4), (6, 29, 31, 2, 8), (2, 512, 512, 0, 2),
+    (4, 513, 513, 0, 2), (2, 363, 367, 1, 3), (6, 259, 257, 2, 4),
+    (2, 1801, 1203, 0, 2), (2, 1449, 733, 1, 2), (2, 751, 749, 2, 2),
+    (2, 2063, 2049, 0, 1), (2, 1451, 1449, 1, 1), (2, 1025, 1031, 2, 1),
+    # without secondary rays a sixteenth of the samples takes each of them
+    (1, 128, 128, 0, 4), (1, 131, 127, 0, 4), (2, 363, 367, 0, 0), (4, 363, 367, 1, 0),
+])
+def test_gpu_one_kernel_lanes_per_sample(device, config, x, y, fsaa, depth):
+    """However many lanes trace a sample, and over ragged tiles, the frame and
+    the first-hit ids are those of the level pipeline."""
+    device.set_fsaa(fsaa)
+    hs = HostScene(config, 51, x, y, fsaa, depth)
+    try:
+        want, wid = device.render_tables(hs.tables, hs.fd, want_ids=True)
+        device.set_path(qrhip.PATH_ONE_KERNEL)
+        got, gid = device.render_tables(hs.tables, hs.fd, want_ids=True)
+    finally:
+        device.set_path(qrhip.PATH_LEVELS)
+        hs.close()
+    assert np.array_equal(got, want)
+    assert np.array_equal(gid, wid)
