@@ -59,7 +59,8 @@ int  qrhip_device_get_fsaa_max(qrhip_dev *dev);
 
 /* Tracing path for frames rendered on this device (no counterpart in
  * QuadRay, which has one CPU path): QRHIP_PATH_LEVELS, the default, traces
- * the Whitted tree level by level over compacted ray queues;
+ * the Whitted tree level by level over compacted ray queues (a frame without
+ * secondary rays has one level, and most such frames are one kernel);
  * QRHIP_PATH_ONE_KERNEL traces each sample's whole tree in one kernel (also
  * used for scenes with more than 32 lights).  Both give identical frames. */
 #define QRHIP_PATH_LEVELS      0

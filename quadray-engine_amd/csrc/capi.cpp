@@ -36,10 +36,20 @@ int hip_fail(hipError_t e, const char *what)
 hipError_t launch_frame(const qrhip_dev *d, qr_wf_state *wf, const qr_device_tables *t,
                         const qr_frame_desc *fd, uint32_t *frame, int32_t *ids)
 {
-    if (d->path == QRHIP_PATH_LEVELS && t->n_lgt <= qr_wf_max_lights())
+    /* a frame without secondary rays has one level and no tree to spread over
+     * queues, so one kernel draws it.  us, levels -> one kernel: 6 surfaces,
+     * one light, 800x480 46 -> 14, 1920x1080 at 4 samples 613 -> 162; 77
+     * surfaces, 4 lights, 64x64 95 -> 47, 1920x1080 at 4 samples 914 -> 561;
+     * 397 surfaces 2912 -> 2578.  With 1165 surfaces the walks' compacted
+     * shadow rays win once the chip is full: 1280x720 1350 -> 1475, but
+     * 300x200 655 -> 357 */
+    const uint64_t n = (uint64_t)fd->x_res * (uint64_t)fd->y_res * (uint64_t)(1 << fd->fsaa);
+    const bool one_level = !qr_frame_has_tree(t, fd) && (t->n_surf <= 512 || n <= (1u << 17));
+    if (d->path == QRHIP_PATH_LEVELS && t->n_lgt <= qr_wf_max_lights() && !one_level)
     {
         return qr_wf_launch(wf, t, fd, frame, ids, d->stream);
     }
+    if (wf != nullptr) qr_wf_skip(wf);
     return qr_launch_whitted(t, fd, frame, ids, d->stream);
 }
 

@@ -8,8 +8,8 @@
  * 5160-5277) becomes an explicit per-lane stack of pending tree nodes;
  * colours are accumulated bottom-up in QuadRay's order.
  * The level-by-level pipeline (tracer_wf.hip) is the default path; this
- * kernel serves scenes beyond that pipeline's light-mask limit, and callers
- * that cannot allocate.
+ * kernel serves frames without secondary rays, scenes beyond that pipeline's
+ * light-mask limit, and callers that cannot allocate.
  *
  * Its time is that of its longest waves, whose lanes' trees are walked node
  * by node while the rest of the chip has run dry (vector issue was 4% busy
@@ -23,8 +23,11 @@
  *
  * Times, one pixel per lane before -> now: 640x360 at 2 samples, depth 4:
  * 2.55 -> 0.61 ms; 641x359 at 4, depth 8: 102 -> 11.0; 1281x719 at 2:
- * 9.6 -> 3.6; 64x64: 1.12 -> 0.31; 1920x1080 at 4: 5.3 -> 1.8; 800x480
- * without secondary rays: 0.020 -> 0.019.
+ * 9.4 -> 3.3; 64x64: 1.12 -> 0.29; 1920x1080 at 4: 5.2 -> 1.8.
+ *
+ * A frame without secondary rays needs no stack (1360 bytes of scratch and
+ * 20 registers): 800x480 with one light 20 -> 14 us, 1920x1080 at 4 samples
+ * 247 -> 162, with four lights 741 -> 561.
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -49,6 +52,65 @@ __device__ __forceinline__ Ray child(const Node &nd, int which)
     return c;
 }
 
+/* the colour of a hit, its lights' shadow rays tested by the SPLIT lanes that
+ * hold the sample, one each at a time */
+template <int SPLIT>
+__device__ __forceinline__ V3 hit_colour(const Scene &sc, const qr_frame_desc &fd, const Ray &ray,
+                                         const Hit &h, const V3 &nrm)
+{
+    const int sub = (int)(threadIdx.x & (SPLIT - 1));
+    const int group = __lane_id() & ~(SPLIT - 1);
+    V3 tex;
+    bool lit;
+    V3 col = shade_base(sc, fd, h, tex, lit);
+    for (int l0 = 0; lit && l0 < sc.n_lgt; l0 += SPLIT)
+    {
+        /* this lane's light of the next four, then all four added in
+         * their order */
+        const int li = l0 + sub;
+        Ray sr;
+        bool vis = li < sc.n_lgt && 0.0f < light_vec(sc.lgt[li], h.hit, nrm, sr.dir);
+        if (vis)
+        {
+            sr.org = h.hit;
+            sr.t_min = 0.0f;
+            sr.t_max = sc.lgt[li].t_max;
+            sr.flags = h.side | FLAG_SHAD;
+            sr.origin = h.srf;
+            sr.oloc = h.loc;
+            sr.depth = 0;
+            Hit sh;
+            vis = !walk<true>(sc, sr, sh);
+        }
+        const uint32_t four = (uint32_t)(lanes(vis) >> group);
+        for (int k = 0; k < SPLIT && l0 + k < sc.n_lgt; k++)
+        {
+            if (!((four >> k) & 1u)) continue;
+            const QC qr_light &l = sc.lgt[l0 + k];
+            V3 L;
+            const float dot = light_vec(l, h.hit, nrm, L);
+            shade_light(sc, l, ray.dir, h, nrm, tex, L, dot, col);
+        }
+    }
+    return col;
+}
+
+/* one camera sample of a frame without secondary rays */
+template <int SPLIT>
+__device__ V3 trace_camera(const Scene &sc, const qr_frame_desc &fd, const Ray &ray,
+                           int32_t *hit_id)
+{
+    Hit h;
+    if (!walk<false>(sc, ray, h))
+    {
+        *hit_id = -1;
+        return V3{0.0f, 0.0f, 0.0f};
+    }
+    *hit_id = (sc.srf[h.srf].id << 1) | h.side;
+    hit_info(sc, ray, h);
+    return hit_colour<SPLIT>(sc, fd, ray, h, normal_at(sc, h));
+}
+
 /* one camera sample through the whole Whitted tree: a node waits on the
  * stack for its refraction child, then its reflection child, and folds each
  * result into its colour as QuadRay's TR_mix / RF_mix do */
@@ -56,8 +118,6 @@ template <int SPLIT>
 __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
                            int32_t *hit_id)
 {
-    const int sub = (int)(threadIdx.x & (SPLIT - 1));
-    const int group = __lane_id() & ~(SPLIT - 1);
     Node stk[MAX_STACK];
     int sp = 0;
     V3 ret = {0.0f, 0.0f, 0.0f};
@@ -79,39 +139,7 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
             hit_info(sc, ray, h);
             const V3 nrm = normal_at(sc, h);
             Node &nd = stk[sp];
-            V3 tex;
-            bool lit;
-            V3 col = shade_base(sc, fd, h, tex, lit);
-            for (int l0 = 0; lit && l0 < sc.n_lgt; l0 += SPLIT)
-            {
-                /* this lane's light of the next four, then all four added in
-                 * their order */
-                const int li = l0 + sub;
-                Ray sr;
-                bool vis = li < sc.n_lgt && 0.0f < light_vec(sc.lgt[li], h.hit, nrm, sr.dir);
-                if (vis)
-                {
-                    sr.org = h.hit;
-                    sr.t_min = 0.0f;
-                    sr.t_max = sc.lgt[li].t_max;
-                    sr.flags = h.side | FLAG_SHAD;
-                    sr.origin = h.srf;
-                    sr.oloc = h.loc;
-                    sr.depth = 0;
-                    Hit sh;
-                    vis = !walk<true>(sc, sr, sh);
-                }
-                const uint32_t four = (uint32_t)(lanes(vis) >> group);
-                for (int k = 0; k < SPLIT && l0 + k < sc.n_lgt; k++)
-                {
-                    if (!((four >> k) & 1u)) continue;
-                    const QC qr_light &l = sc.lgt[l0 + k];
-                    V3 L;
-                    const float dot = light_vec(l, h.hit, nrm, L);
-                    shade_light(sc, l, ray.dir, h, nrm, tex, L, dot, col);
-                }
-            }
-            nd.col = col;
+            nd.col = hit_colour<SPLIT>(sc, fd, ray, h, nrm);
             node_children(sc, ray, h, nrm, nd);
             if (nd.todo & 1)
             {
@@ -183,10 +211,13 @@ __host__ __device__ constexpr int tile_h(int ns)
     return 1 << (log2i(64 / SPLIT / ns) / 2);
 }
 
-/* four waves per workgroup, their tiles side by side; a pixel's samples in neighbouring
+/* without a tree: 6 waves per SIMD spare a full chip more than their 36 bytes
+ * of spills cost (397 surfaces at 1920x1080 and 4 samples, 5 -> 6 waves:
+ * 2784 -> 2578 us); a frame that leaves it idle gains nothing by them (64x64
+ * 47 -> 49).  Four waves per workgroup, their tiles side by side; a pixel's samples in neighbouring
  * groups of SPLIT lanes */
-template <int SPLIT>
-__global__ void __launch_bounds__(256)
+template <int SPLIT, bool TREE>
+__global__ void __launch_bounds__(256, !TREE && SPLIT == 1 ? 6 : 4)
 whitted_kernel(Scene sc, qr_frame_desc fd, int ns, uint32_t *__restrict__ frame,
                int32_t *__restrict__ ids)
 {
@@ -225,7 +256,7 @@ whitted_kernel(Scene sc, qr_frame_desc fd, int ns, uint32_t *__restrict__ frame,
         r.oloc = V3{0.0f, 0.0f, 0.0f};
         r.depth = fd.depth;
         int32_t id;
-        c = trace_sample<SPLIT>(sc, fd, r, &id);
+        c = TREE ? trace_sample<SPLIT>(sc, fd, r, &id) : trace_camera<SPLIT>(sc, fd, r, &id);
         c.x = c.x < 1.0f ? c.x : 1.0f;
         c.y = c.y < 1.0f ? c.y : 1.0f;
         c.z = c.z < 1.0f ? c.z : 1.0f;
@@ -238,14 +269,14 @@ whitted_kernel(Scene sc, qr_frame_desc fd, int ns, uint32_t *__restrict__ frame,
     if (in && first && k == 0) frame[(ptrdiff_t)y * fd.x_row + x] = px;
 }
 
-template <int SPLIT>
+template <int SPLIT, bool TREE>
 void launch(const Scene &sc, const qr_frame_desc &fd, int ns, uint32_t *frame, int32_t *ids,
             hipStream_t stream)
 {
     const int tw = 4 * tile_w<SPLIT>(ns), th = tile_h<SPLIT>(ns);
     const unsigned nx = (unsigned)((fd.x_res - 1) / tw + 1), ny = (unsigned)((fd.y_res - 1) / th + 1);
     const unsigned gy = ny < 65535u ? ny : 65535u;
-    hipLaunchKernelGGL(whitted_kernel<SPLIT>, dim3(nx, gy, (ny + gy - 1) / gy), dim3(256), 0, stream,
+    hipLaunchKernelGGL((whitted_kernel<SPLIT, TREE>), dim3(nx, gy, (ny + gy - 1) / gy), dim3(256), 0, stream,
                        sc, fd, ns, frame, ids);
 }
 
@@ -267,11 +298,16 @@ hipError_t qr_launch_whitted(const qr_device_tables *t, const qr_frame_desc *fd,
      * 0.96 2.68; at 2 samples 1.49 1.30 1.51 5.41; at 4 1.80 1.88 2.99 9.75;
      * without secondary rays, 64x64 0.148 0.092 0.060 0.048; 640x360 at 2
      * 0.089 0.089 0.125 0.431 (8 lanes lie between 4 and 16) */
-    const bool tree = t->spawns && fd->depth > 0;
-    const uint64_t n = (uint64_t)fd->x_res * (uint64_t)fd->y_res * (uint64_t)ns * (tree ? 1u : 16u);
-    if (n <= (1u << 18)) launch<16>(sc, *fd, ns, frame, ids, stream);
-    else if (n <= (1u << 21)) launch<4>(sc, *fd, ns, frame, ids, stream);
-    else if (n <= (1u << 22)) launch<2>(sc, *fd, ns, frame, ids, stream);
-    else launch<1>(sc, *fd, ns, frame, ids, stream);
+    const uint64_t n = (uint64_t)fd->x_res * (uint64_t)fd->y_res * (uint64_t)ns;
+    if (!qr_frame_has_tree(t, fd))
+    {
+        if (n <= (1u << 14)) launch<16, false>(sc, *fd, ns, frame, ids, stream);
+        else if (n <= (1u << 17)) launch<4, false>(sc, *fd, ns, frame, ids, stream);
+        else launch<1, false>(sc, *fd, ns, frame, ids, stream);
+    }
+    else if (n <= (1u << 18)) launch<16, true>(sc, *fd, ns, frame, ids, stream);
+    else if (n <= (1u << 21)) launch<4, true>(sc, *fd, ns, frame, ids, stream);
+    else if (n <= (1u << 22)) launch<2, true>(sc, *fd, ns, frame, ids, stream);
+    else launch<1, true>(sc, *fd, ns, frame, ids, stream);
     return hipGetLastError();
 }

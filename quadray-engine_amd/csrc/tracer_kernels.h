@@ -262,6 +262,12 @@ static inline int qr_side_spawns(uint32_t props)
     return (props & QR_PROP_REFLECT) != 0 || (props & QR_PROP_OPAQUE) == 0;
 }
 
+/* can a ray of the frame have children? */
+static inline bool qr_frame_has_tree(const qr_device_tables *t, const qr_frame_desc *fd)
+{
+    return t->spawns != 0 && fd->depth > 0;
+}
+
 /* hot[i] from srf[i] for every record, on the device */
 hipError_t qr_dev_surfaces(const qr_surface *srf, int n, qr_dev_surf *hot, hipStream_t stream);
 
@@ -337,6 +343,8 @@ hipError_t qr_wf_launch(qr_wf_state *s, const qr_device_tables *t,
 /* after the stream finished the frame: 0 if it is complete, 1 if a queue
  * overflowed (queues are grown; trace the frame again) */
 int        qr_wf_check(qr_wf_state *s, qr_wf_stats *stats);
+/* the frame launched last went another way: there is nothing to check */
+void       qr_wf_skip(qr_wf_state *s);
 
 /* Batches: many frames, each with its own queues (state), tables, camera,
  * resolution, anti-aliasing and depth, traced by one launch per stage.  The

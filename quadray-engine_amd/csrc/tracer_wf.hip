@@ -1561,6 +1561,11 @@ hipError_t qr_wf_launch(qr_wf_state *s, const qr_device_tables *t,
     return qr_wf_batch_launch(s->own, &it, 1, stream);
 }
 
+void qr_wf_skip(qr_wf_state *s)
+{
+    if (s->own != nullptr) s->own->nfr = 0;
+}
+
 int qr_wf_check(qr_wf_state *s, qr_wf_stats *stats)
 {
     if (s->own == nullptr) return 0;

@@ -366,3 +366,41 @@ def test_gpu_one_kernel_lanes_per_sample(device, config, x, y, fsaa, depth):
         hs.close()
     assert np.array_equal(got, want)
     assert np.array_equal(gid, wid)
+
+
+@pytest.mark.parametrize("config,x,y,fsaa,depth", [
+    # without secondary rays: 16, 4 and 1 lanes to a sample, ragged tiles, one
+    # light and four, and either side of the size a dense scene changes path at
+    (1, 1, 1, 2, 4), (1, 127, 129, 0, 4), (1, 131, 127, 0, 4), (1, 181, 187, 1, 4),
+    (1, 363, 367, 0, 4), (2, 257, 259, 1, 0), (4, 37, 23, 2, 0), (4, 91, 95, 2, 0),
+    (11, 363, 361, 0, 0), (11, 363, 363, 0, 0),
+])
+def test_gpu_frames_without_secondary_rays(path_dev, config, x, y, fsaa, depth):
+    hs = HostScene(config, 52, x, y, fsaa, depth)
+    try:
+        want, wid, flags, _, _ = hs.oracle(want_ids=True)
+        got, gid = path_dev.render_tables(hs.tables, hs.fd, want_ids=True)
+    finally:
+        hs.close()
+    assert_frame_exact(got, want, "frame")
+    assert not np.any((gid != wid) & (flags == 0))
+
+
+def test_gpu_depth_changes_path_between_frames(device):
+    """A scene's frames with and without secondary rays in turn: queues that
+    overflow in the one kind leave nothing to check in the other."""
+    w, s = gpu_scene(device, 6, 53, 160, 90, 2, 8)
+    got = []
+    try:
+        for depth in (0, 8, 0, 8):
+            s.set_depth(depth)
+            got.append(s.render(0).copy())
+    finally:
+        s.destroy()
+        w.close()
+    for depth, frame in zip((0, 8, 0, 8), got):
+        hs = HostScene(6, 53, 160, 90, 2, depth)
+        try:
+            assert_frame_exact(frame, hs.oracle()[0], depth)
+        finally:
+            hs.close()
