@@ -280,8 +280,9 @@ int  qrhip_batch_tune(qrhip_batch *b, int reps, int *best, float *ms);
  * admitted frame is split into chunks (runs of level-0 tiles); each step
  * takes, within a budget of camera samples, a chunk of the oldest request in
  * flight and then chunks of the requests with the least work left, traces
- * the Whitted chunks as one batch (one launch per pipeline stage) and one
- * pass of each path-traced chunk, and returns the frames that finished.
+ * the Whitted chunks as one batch (one launch per pipeline stage) and a
+ * pass of each path-traced chunk (without a time budget, as many passes as
+ * the step's samples allow), and returns the frames that finished.
  * Steps are pipelined (the next is launched before the last is retired).
  * Requests that arrive during a step join the next one, so a small frame
  * does not wait for a large one to finish.  A frame is the same whatever

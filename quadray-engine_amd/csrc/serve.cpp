@@ -429,7 +429,7 @@ void qrhip_server::account(StepCtx &c)
     }
 }
 
-/* enqueue a step: its Whitted chunks as one batch, then one pass of each
+/* enqueue a step: its Whitted chunks as one batch, then the passes of each
  * path-traced chunk, then the step's event */
 hipError_t qrhip_server::launch(StepCtx &c)
 {

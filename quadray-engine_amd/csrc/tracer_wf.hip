@@ -708,7 +708,7 @@ __device__ __forceinline__ void shading(const QC Frame &a, int L, uint32_t i)
 }
 
 /* stage 0: nearest walks of the camera samples */
-/* six waves per SIMD (80 VGPRs, 6 spilled; 1% faster per frame than five) */
+/* six waves per SIMD (79 VGPRs, none spilled; 1% faster per frame than five) */
 template <int R>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(6, 6))) k_walk0(Batch b)
 {
@@ -729,7 +729,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(6, 6)))
 }
 
 /* a stage of shadow walks alone (level b.sl) */
-/* eight waves per SIMD (64 VGPRs, 3 spilled outside the inner loops): the
+/* eight waves per SIMD (64 VGPRs, none spilled): the
  * extra waves hide more of the walk's scalar-load latency, and leave room
  * for level 1's nearest walks beside it (measured per frame: 1.2% faster
  * than seven waves, 2.5% faster than six) */
@@ -746,7 +746,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8, 8)))
 }
 
 /* a stage of nearest walks alone (level b.wl >= 1) */
-/* five waves per SIMD (93 VGPRs) */
+/* five waves per SIMD (87 VGPRs) */
 template <int R>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(5, 5))) k_walk(Batch b)
 {
@@ -785,7 +785,7 @@ __global__ void __launch_bounds__(WG) k_shading(Batch b)
 /* a stage of two or three kinds of work: per frame, the shadow walks of
  * level b.sl, then the nearest walks of level b.wl >= 1, then the shading of
  * level b.fl >= 1 (shadow walks first measured 1.7% faster per frame) */
-/* seven waves per SIMD (72 VGPRs, 11 spilled): the deeper levels' short
+/* seven waves per SIMD (72 VGPRs, 40 bytes spilled): the deeper levels' short
  * queues are latency bound (measured per frame: 1.775 ms at seven, 1.816
  * at six, 1.807 at eight with 29 spilled; five was 4% slower than six) */
 template <int R>
