@@ -248,6 +248,7 @@ __device__ __forceinline__ const QC qr_dev_surf *surf_at(const Scene &sc, uint32
 __device__ __forceinline__ V3 xform(const SurfHead &s, const QC qr_dev_surf *p, const V3 &d)
 {
     if ((s.flags & QR_DS_TRM) == QR_DS_TRM_DIAG) return xform_diag(s.td, d);
+    if ((s.flags & QR_DS_TRM) == 0 && p->info == QR_DI_TRM_DIAG) return xform_diag(s.td, d);
     return xform_full(s.td, ldk<SurfOff>(p->to).to, d);
 }
 
@@ -779,7 +780,7 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
              * of list order) */
             if (e > cache_last || e < cache_first) cache_last = -1;
             V3 rr, dd;
-            if (cache_last >= 0 && (s.flags & QR_DS_NODE) == 0)
+            if (cache_last >= 0 && (s.flags & QR_DS_SOLO) == 0)
             {
                 dd = sub3(node_o, s.pos);
                 rr = node_d;
@@ -802,7 +803,7 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
                         dd = xform_diag(s.td, dd);
                         rr = xform_diag(s.td, rr);
                     }
-                    if (s.flags & QR_DS_NODE)
+                    if (s.flags & QR_DS_SOLO)
                     {
                         /* a transform node (never a ray's origin) opens its
                          * group, whose end its step holds: the ray in the
@@ -821,7 +822,22 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
                         s_gb[6][tid] = gb.hx;
                         s_gb[7][tid] = gb.hy;
                         s_gb[8][tid] = gb.hz;
+                        /* (were the node a surface in world coordinates) */
+                        if (!(s.flags & QR_DS_SHIFT)) rr = r.dir;
                     }
+                }
+                else if (cache_last >= 0)
+                {
+                    /* inside a group, but in world coordinates (caller
+                     * tables alone): the origin register holds what the node
+                     * left, or the ray's own surface's local hit; a node
+                     * without a transform leaves it its own */
+                    if ((sp->info & QR_DI_NODE) == 0)
+                    {
+                        dd = pick(soff == org_off, r.oloc, node_o);
+                        if (e == cache_last) cache_last = -1;
+                    }
+                    node_o = dd;
                 }
             }
             const uint64_t same = lanes(soff == org_off);
@@ -977,11 +993,11 @@ __device__ void hit_info(const Scene &sc, const Ray &r, Hit &h)
     V3 dd, rr;
     bool cached = false;
     const int node = s.trnode;
-    if ((flags & QR_DS_NODE) == 0 && node >= 0 && node != h.srf)
+    if ((s.info & QR_DI_NODE) == 0 && node >= 0 && node != h.srf)
     {
         const QC qr_dev_surf &n = sc.hot[node];
         const uint32_t nf = n.flags;
-        if ((nf & QR_DS_NODE) != 0 && (nf & QR_DS_TRM) != 0)
+        if ((nf & QR_DS_SOLO) != 0 && (nf & QR_DS_TRM) != 0)
         {
             const float nd[3] = {n.td[0], n.td[1], n.td[2]};
             const V3 d = sub3(r.org, n.pos);
@@ -1088,15 +1104,15 @@ __device__ V3 normal_at(const Scene &sc, const Hit &h)
         float inv = fxor(rsq(rr), ts);
         n = V3{l.x * inv, l.y * inv, l.z * inv};
     }
-    if ((flags & QR_DS_TRM) == 0) return n;
+    if ((s.info & QR_DI_TRM) == 0) return n;
 
     const QC qr_dev_surf &t = sc.hot[s.trnode];
-    const uint32_t trm = t.flags & QR_DS_TRM;
+    const uint32_t trm = t.info & QR_DI_TRM;
     float x = t.td[0] * n.x;
     float y = t.td[1] * n.y;
     float z = t.td[2] * n.z;
     bool renorm = true;
-    if (trm != QR_DS_TRM_DIAG)
+    if (trm != QR_DI_TRM_DIAG)
     {
         /* the transposed matrix: to holds 01 02 10 12 20 21 */
         x = x + t.to[2] * n.y;
@@ -1105,7 +1121,7 @@ __device__ V3 normal_at(const Scene &sc, const Hit &h)
         y = y + t.to[5] * n.z;
         z = z + t.to[1] * n.x;
         z = z + t.to[3] * n.y;
-        renorm = trm != QR_DS_TRM_ROT;
+        renorm = trm != QR_DI_TRM_ROT;
     }
     if (renorm)
     {

@@ -73,14 +73,18 @@ typedef struct qr_dev_surf
     float    to[6];             /* off its diagonal: 01 02 10 12 20 21 */
     int32_t  clip_beg, clip_cnt;
     int32_t  trnode;            /* record of the transform node, -1: none */
-    int32_t  pad;
+    uint32_t info;              /* QR_DI_* */
 } qr_dev_surf;
 #define QR_DS_CLASS     0x7u            /* QR_DC_* */
-#define QR_DS_SHIFT     0x8u            /* traced in its node's frame */
-#define QR_DS_TRM       0x30u           /* any transform; bits: none, diagonal, */
-#define QR_DS_TRM_DIAG  0x10u           /* rotation, rotation and scale */
-#define QR_DS_TRM_ROT   0x20u
-#define QR_DS_NODE      0x40u           /* a transform node (an array) */
+#define QR_DS_SHIFT     0x8u            /* traced in its node's or its own frame */
+#define QR_DS_TRM       0x30u           /* the transform into that frame (a node's: */
+#define QR_DS_TRM_DIAG  0x10u           /* its group's); bits: none, diagonal,
+                                           rotation, rotation and scale */
+#define QR_DS_SOLO      0x40u           /* not in an open group's frame: a transform
+                                           node, or a surface without "shift",
+                                           which is traced in world coordinates
+                                           (and has no QR_DS_TRM, whatever
+                                           transform its record holds) */
 #define QR_DS_APEX      0x80u
 #define QR_DS_APEX_TWO  0x100u          /* apex kind 2 (two planes) */
 #define QR_DS_CMIN_BIT  9               /* bit 9 + a: axis a has a min clip */
@@ -93,6 +97,13 @@ typedef struct qr_dev_surf
 #define QR_DS_SHADOW_BIT 27             /* bit 27 + side: it casts shadows */
 #define QR_DS_NRM_BIT   29              /* two bits: nrm_kind 1, 2 or 3 */
 #define QR_DS_OWN_LIST  0x80000000u     /* rays leaving it walk a list of its own */
+/* what the walk's loop does not read: the record's transform as it stands
+ * (normals turn by their node's), and whether it is a transform node (an
+ * array) */
+#define QR_DI_TRM       0x3u
+#define QR_DI_TRM_DIAG  0x1u
+#define QR_DI_TRM_ROT   0x2u
+#define QR_DI_NODE      0x4u
 /* classes: QR_SOLVE_* with the quadrics that need fewer operations apart.
  * x - (+0) and x * 1 are x for every x, so those are the same roots. */
 #define QR_DC_PLANE     1
@@ -124,9 +135,10 @@ static inline QR_HD void qr_dev_surf_of(const qr_surface *r, int n_surf, qr_dev_
         if (pure) f = unit ? QR_DC_SPHERE : QR_DC_PURE;
     }
     if (r->shift != 0) f |= QR_DS_SHIFT;
-    f |= r->trm == 0 ? 0u : r->trm == 1 ? QR_DS_TRM_DIAG : r->trm == 2 ? QR_DS_TRM_ROT
-                                                                       : QR_DS_TRM;
-    if (r->tag < 0) f |= QR_DS_NODE;
+    const uint32_t trm = r->trm == 0 ? 0u : r->trm == 1 ? QR_DI_TRM_DIAG
+                                          : r->trm == 2 ? QR_DI_TRM_ROT : QR_DI_TRM;
+    if (r->shift != 0 || r->tag < 0) f |= trm * QR_DS_TRM_DIAG;
+    if (r->shift == 0 || r->tag < 0) f |= QR_DS_SOLO;
     if (r->apex != 0) f |= QR_DS_APEX;
     if (r->apex == 2) f |= QR_DS_APEX_TWO;
     f |= ((uint32_t)r->cmin_on & 7u) << QR_DS_CMIN_BIT;
@@ -174,7 +186,7 @@ static inline QR_HD void qr_dev_surf_of(const qr_surface *r, int n_surf, qr_dev_
     d->clip_beg = r->clip_beg;
     d->clip_cnt = r->clip_cnt;
     d->trnode = r->trnode >= 0 && r->trnode < n_surf ? r->trnode : -1;
-    d->pad = 0;
+    d->info = trm | (r->tag < 0 ? QR_DI_NODE : 0u);
 }
 static inline QR_HD void qr_dev_box_step(qr_dev_step *d, int skip_index)
 {

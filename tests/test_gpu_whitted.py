@@ -342,6 +342,72 @@ def test_gpu_root_forms(path_dev, config, seed, d_eps, zero):
     assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
 
 
+def _snapshot(config, seed, x, y, fsaa, depth):
+    hs = HostScene(config, seed, x, y, fsaa, depth)
+    try:
+        return qrhip.tables_snapshot(hs.tables, hs.fd)
+    finally:
+        hs.close()
+
+
+def _render_every_way(path_dev, t):
+    """A table's (frame, ids) through the allocating and the no-alloc entry
+    points."""
+    return [path_dev.render_tables(t.ptr, t.fd, want_ids=True),
+            path_dev.render_tables_noalloc(t.ptr, t.fd, want_ids=True)]
+
+
+@pytest.mark.parametrize("config,depth", [(1, 0), (1, 4), (9, 0), (9, 5)])
+def test_gpu_world_surfaces_with_a_transform(path_dev, config, depth):
+    """Caller tables whose surfaces are traced in world coordinates (shift 0)
+    though they carry a transform (trm): their transform node, an identity
+    rotation, turns their normals; their own matrix is read by nothing.  The
+    frame and the first-hit ids are those of the tables without transforms."""
+    snap = _snapshot(config, 21, 95, 63, 1, depth)
+    t = qrhip.TablesFromSnapshot(snap)
+    want, ids_o, flags, _, _ = qr_oracle.render(t.ptr, t.fd, want_ids=True)
+    t = qrhip.TablesFromSnapshot(snap)
+    world = [i for i in range(t.tables.n_surf)
+             if t.tables.surfaces[i].tag >= 0 and t.tables.surfaces[i].trm == 0]
+    assert len(world) >= 5
+    rng = np.random.default_rng(config)
+    for k, i in enumerate(world):
+        s = t.tables.surfaces[i]
+        s.trm = 2 if k == 0 else 1 + k % 3
+        s.trnode = world[0]
+        for r in range(3):
+            for c in range(3):
+                s.tc[r][c] = float(r == c) if k == 0 else float(rng.uniform(-2.0, 2.0))
+    for got, ids in _render_every_way(path_dev, t):
+        assert_frame_exact(got, want, f"config {config} depth {depth}")
+        assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
+
+
+@pytest.mark.parametrize("config,depth", [(2, 0), (2, 4), (9, 0), (9, 5)])
+def test_gpu_world_surfaces_in_a_group(path_dev, config, depth):
+    """Caller tables with surfaces traced in world coordinates (shift 0)
+    inside a transform node's group: the ray's direction stays the world's
+    and its origin is the one the node left, as in QuadRay's list walk; bit
+    for bit the oracle's frame.  (No culling program: its local boxes are for
+    surfaces in the node's frame.)"""
+    snap = _snapshot(config, 22, 93, 59, 1, depth)
+    t = qrhip.TablesFromSnapshot(snap)
+    t.tables.n_step = t.tables.n_step_any = 0
+    changed = 0
+    for i in range(t.tables.n_surf):
+        s = t.tables.surfaces[i]
+        if s.tag >= 0 and s.shift != 0 and s.trnode not in (-1, i):
+            changed += 1
+            if changed % 2 == 1:
+                s.shift = s.trm = s.apex = 0
+                s.trnode = -1
+    assert changed >= 4
+    want, ids_o, flags, _, _ = qr_oracle.render(t.ptr, t.fd, want_ids=True)
+    for got, ids in _render_every_way(path_dev, t):
+        assert_frame_exact(got, want, f"config {config} depth {depth}")
+        assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
+
+
 @pytest.mark.parametrize("config,x,y,fsaa,depth", [
     # 16 lanes to a sample: the smallest frame, ragged edges of every tile
     # shape, the largest number of samples; then 4, 2 and 1 lanes
