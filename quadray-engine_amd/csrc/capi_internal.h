@@ -227,6 +227,7 @@ inline ProgramInputs program_inputs(const qr::Engine &eng)
 struct DevTables
 {
     DevBuf srf, hot, mat, lgt, clp, elem, tex, step, step_any, refit_in, refit_box;
+    bool   hot_valid = false;       /* hot holds srf's records as the walks read them */
     DevBuf geom, expect;            /* the device update stage's inputs */
     uint32_t *flag_host = nullptr;  /* pinned: set by the device's kernels */
     uint64_t expect_build = 0;      /* the build "expect" holds the flags of */
@@ -339,6 +340,16 @@ struct DevTables
                        memcmp(sent[i].data(), it.src, it.n) != 0);
             if (send[i]) total += (it.n + 255) & ~(size_t)255;
         }
+        /* the walks' form of the surfaces: not srf's from here on until its
+         * conversion is enqueued, whichever call in between fails */
+        void *hot_was = hot.ptr;
+        if (send[2]) hot_valid = false;
+        if ((e = hot.reserve(sizeof(qr_dev_surf) * (size_t)h.n_surf)) != hipSuccess)
+        {
+            hot_valid = false;
+            return e;
+        }
+        if (hot.ptr != hot_was) hot_valid = false;
         const size_t rbytes = refit != nullptr ? sizeof(qr_refit_elem) * (size_t)refit->n_elem
                                                : 0;
         total += (rbytes + 255) & ~(size_t)255;
@@ -362,13 +373,12 @@ struct DevTables
             }
             if ((e = stage.end(st)) != hipSuccess) return e;
         }
-        if ((e = hot.reserve(sizeof(qr_dev_surf) * (size_t)h.n_surf)) != hipSuccess) return e;
-        if (send[2] && (e = qr_dev_surfaces((const qr_surface *)srf.ptr, h.n_surf,
-                                            (qr_dev_surf *)hot.ptr, st)) != hipSuccess)
+        if (!hot_valid && (e = qr_dev_surfaces((const qr_surface *)srf.ptr, h.n_surf,
+                                               (qr_dev_surf *)hot.ptr, st)) != hipSuccess)
         {
-            sent[2].clear();
             return e;
         }
+        hot_valid = true;
         t.surfaces = (qr_surface *)srf.ptr;
         t.hot = (qr_dev_surf *)hot.ptr;
         t.materials = (qr_material *)mat.ptr;
@@ -409,6 +419,7 @@ struct DevTables
         flag_host = nullptr;
         stage.release();
         for (std::vector<uint8_t> &v : sent) v.clear();
+        hot_valid = false;
         build_on_dev = 0;
         expect_build = 0;
     }
@@ -477,8 +488,9 @@ struct DevTables
         if (send_lgt)
         {
             const uint8_t *src = (const uint8_t *)h.lights;
-            sent[4].assign(src, src + lbytes);
+            sent[4].clear();
             if ((e = stage.copy(lgt.ptr, src, lbytes, st)) != hipSuccess) return e;
+            sent[4].assign(src, src + lbytes);
         }
         if ((e = stage.end(st)) != hipSuccess) return e;
         if (send_expect) expect_build = build_on_dev;
@@ -490,6 +502,10 @@ struct DevTables
                 t.spawns = 1;
             }
         }
+        /* from here on the device holds records, materials and boxes no host
+         * copy has, also if a call below fails */
+        for (int i : {0, 1, 2, 3}) sent[i].clear();
+        hot_valid = false;
         /* (the last update's kernels are done: it waited for them) */
         *flag_host = 0u;
         e = qr_update_records((const qr_geom *)geom.ptr, h.n_surf, (const qr_clip *)clp.ptr,
@@ -497,6 +513,7 @@ struct DevTables
                               (qr_material *)mat.ptr, (qr_refit_elem *)refit_in.ptr,
                               (const int32_t *)expect.ptr, flag_host, st);
         if (e != hipSuccess) return e;
+        hot_valid = true;
         e = qr_refit_programs((qr_dev_step *)step.ptr, dev_n_step,
                               any ? (qr_dev_step *)step_any.ptr : nullptr, any ? dev_n_any : 0,
                               (const qr_refit_elem *)refit_in.ptr, n_elem,
@@ -504,8 +521,6 @@ struct DevTables
                               (float *)refit_box.ptr, st);
         if (e != hipSuccess) return e;
         if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-        /* the device now holds records, materials and boxes no host copy has */
-        for (int i : {0, 1, 2, 3}) sent[i].clear();
         refits++;
         *ok = *flag_host == 0u;
         return hipSuccess;

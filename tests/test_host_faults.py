@@ -1,0 +1,31 @@
+"""The library's host code when the HIP runtime fails or a thread cannot be
+had: C++ programs that compile it with the runtime's calls on host memory
+(tests/cpp/hip_host.h), so every call can be made to fail without a device."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "quadray-engine_amd", "csrc")
+
+
+def build(out, name, sources):
+    exe = str(out / name)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Wno-unused-function",
+                    "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "include"), "-I", CSRC,
+                    os.path.join(ROOT, "tests", "cpp", name + ".cpp")] +
+                   [os.path.join(CSRC, s) for s in sources] + ["-lpthread", "-o", exe],
+                   check=True)
+    return exe
+
+
+def run(exe, *args):
+    res = subprocess.run([exe, *args], capture_output=True, text=True, timeout=120)
+    assert res.returncode == 0, (res.returncode, res.stdout[-2000:], res.stderr[-2000:])
+    return res.stdout
+
+
+def test_tables_after_a_failed_upload(tmp_path):
+    """Whichever call of an upload or of a device update fails, the next
+    upload leaves every device table current: none is taken for sent."""
+    print(run(build(tmp_path, "upload_faults", ["engine.cpp", "image.cpp"])))
