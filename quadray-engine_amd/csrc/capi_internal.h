@@ -271,6 +271,9 @@ struct DevTables
                 return e;
             }
             if ((e = upload_rest(h, st, n_step, any, ref, false, in)) != hipSuccess) return e;
+            /* the device then holds boxes no host copy has */
+            sent[0].clear();
+            sent[1].clear();
             if ((e = qr_refit_programs((qr_dev_step *)step.ptr, h.n_step,
                                        any ? (qr_dev_step *)step_any.ptr : nullptr,
                                        any ? h.n_step_any : 0,
@@ -280,9 +283,6 @@ struct DevTables
             {
                 return e;
             }
-            /* the device now holds boxes no host copy has */
-            sent[0].clear();
-            sent[1].clear();
             refits++;
             return hipSuccess;
         }
@@ -303,10 +303,14 @@ struct DevTables
         }
         /* any-hit walks use the nearest-hit program when they have none */
         if (any) dev_steps(h.steps_any, h.n_step_any, ref, h.elems, h.surfaces, dstep_any);
+        /* no build's programs until these are enqueued: a refit of programs
+         * that never arrived would be walked */
+        build_on_dev = 0;
+        if ((e = upload_rest(h, st, n_step, any, ref, true, nullptr)) != hipSuccess) return e;
         build_on_dev = in != nullptr ? in->build : 0;
         dev_n_step = n_step;
         dev_n_any = any ? h.n_step_any : 0;
-        return upload_rest(h, st, n_step, any, ref, true, nullptr);
+        return hipSuccess;
     }
 
     /* the tables, and the programs when "programs" (else they are in place);

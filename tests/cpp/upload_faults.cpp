@@ -108,8 +108,8 @@ int main()
      * on (a refit) by the next upload */
     enum { NOTHING, SCENE, OTHER };
     const struct { int first, update, moved; } modes[] = {
-        {NOTHING, 0, 0}, {SCENE, 0, 0},
-        {SCENE, 1, 0}, {OTHER, 0, 0}};
+        {NOTHING, 0, 0}, {NOTHING, 0, 1}, {SCENE, 0, 0}, {SCENE, 0, 1},
+        {SCENE, 1, 0}, {SCENE, 1, 1}, {OTHER, 0, 0}, {OTHER, 0, 1}};
     for (const auto &m : modes)
     {
         for (long call = 0;; call++)
