@@ -12,6 +12,7 @@
 #include <new>
 #include <system_error>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include <hip/hip_runtime.h>
@@ -91,6 +92,22 @@ constexpr size_t DOWN_ROUND = 4u << 20;
 constexpr size_t DOWN_ROUND_MIN = 256u << 10;
 constexpr size_t DOWN_SHARE = 2u << 20;
 constexpr int    DOWN_THREADS = 4;
+
+/* do two frames' buffers share bytes (one buffer given for many frames)?
+ * Threads would copy both at once; downloaded in their order, the later
+ * frame's bytes stay */
+bool shares_memory(const Download &d)
+{
+    std::vector<std::pair<const uint8_t *, size_t>> v;
+    v.reserve(d.ps.size());
+    for (const Download::Piece &p : d.ps) v.emplace_back(p.dst, p.n);
+    std::sort(v.begin(), v.end());
+    for (size_t k = 1; k < v.size(); k++)
+    {
+        if (v[k - 1].first + v[k - 1].second > v[k].first) return true;
+    }
+    return false;
+}
 
 hipError_t enqueue_round(qrhip_batch *b, const Download &d, size_t r)
 {
@@ -174,9 +191,10 @@ hipError_t download(qrhip_batch *b, int k0, int k1)
             return e;
         }
     }
+    const int want = shares_memory(d) ? 1
+                                      : (int)std::min<size_t>(DOWN_THREADS, d.total / DOWN_SHARE);
     if ((e = enqueue_round(b, d, 0)) != hipSuccess) return e;
     if (d.total > d.round && (e = enqueue_round(b, d, 1)) != hipSuccess) return e;
-    const int want = (int)std::min<size_t>(DOWN_THREADS, d.total / DOWN_SHARE);
     std::vector<std::thread> th;
     try
     {

@@ -29,3 +29,11 @@ def test_tables_after_a_failed_upload(tmp_path):
     """Whichever call of an upload or of a device update fails, the next
     upload leaves every device table current: none is taken for sent."""
     print(run(build(tmp_path, "upload_faults", ["engine.cpp", "image.cpp"])))
+
+
+def test_batch_download_into_shared_buffers(tmp_path):
+    """Frames whose requests name the same memory leave what downloads one
+    after another would."""
+    exe = build(tmp_path, "batch_download",
+                ["engine.cpp", "image.cpp", "capi.cpp", "batch.cpp"])
+    run(exe, "shared")
