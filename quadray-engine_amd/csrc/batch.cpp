@@ -8,9 +8,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -195,20 +195,20 @@ hipError_t download(qrhip_batch *b, int k0, int k1)
                                       : (int)std::min<size_t>(DOWN_THREADS, d.total / DOWN_SHARE);
     if ((e = enqueue_round(b, d, 0)) != hipSuccess) return e;
     if (d.total > d.round && (e = enqueue_round(b, d, 1)) != hipSuccess) return e;
-    std::vector<std::thread> th;
+    std::thread th[DOWN_THREADS];
+    int n = 1;
     try
     {
-        th.reserve(DOWN_THREADS);
-        for (int w = 1; w < want; w++)
-            th.emplace_back(download_work, b, std::ref(d), w);
+        for (; n < want; n++) th[n] = std::thread(download_work, b, std::ref(d), n);
     }
-    catch (const std::system_error &)
+    catch (const std::exception &)
     {
-        /* as many threads as there are to be had */
+        /* as many threads as there are to be had (a started one waits for
+         * their number, so none is left behind here) */
     }
-    d.workers = 1 + (int)th.size();
+    d.workers = n;
     download_work(b, d, 0);
-    for (std::thread &t : th) t.join();
+    for (int w = 1; w < n; w++) th[w].join();
     return (hipError_t)d.err.load();
 }
 
@@ -436,7 +436,14 @@ int qrhip_batch_download(qrhip_batch *b, int k)
     if (k >= (int)b->req.size()) return fail(QRHIP_E_ARG, "frame index out of range");
     HIP_TRY(finish(b));
     const int k0 = k < 0 ? 0 : k, k1 = k < 0 ? (int)b->req.size() : k + 1;
-    HIP_TRY(download(b, k0, k1));
+    try
+    {
+        HIP_TRY(download(b, k0, k1));
+    }
+    catch (const std::bad_alloc &)
+    {
+        return fail(QRHIP_E_DEVICE, "out of host memory");
+    }
     return QRHIP_OK;
 }
 

@@ -31,9 +31,11 @@ def test_tables_after_a_failed_upload(tmp_path):
     print(run(build(tmp_path, "upload_faults", ["engine.cpp", "image.cpp"])))
 
 
-def test_batch_download_into_shared_buffers(tmp_path):
+def test_batch_download_into_shared_buffers_and_after_faults(tmp_path):
     """Frames whose requests name the same memory leave what downloads one
-    after another would."""
+    after another would; a download whose allocations, threads or runtime
+    calls fail returns an error or the frames, and the next one the frames."""
     exe = build(tmp_path, "batch_download",
                 ["engine.cpp", "image.cpp", "capi.cpp", "batch.cpp"])
     run(exe, "shared")
+    print(run(exe, "faults"))
