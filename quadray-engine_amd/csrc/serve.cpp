@@ -256,6 +256,8 @@ hipError_t qrhip_server::admit_one(Req *q)
         }
         /* programs built by another scene's engine are never refitted */
         if (sl.dt_scene != q->r.scene) sl.dt.build_on_dev = 0;
+        /* (after an upload that fails the slot holds no scene's tables) */
+        sl.dt_scene = -1;
         const ProgramInputs in = program_inputs(*sc.s->eng);
         if ((e = sl.dt.upload(sc.s->eng->tables(), stream, &in)) != hipSuccess) return e;
         sl.dt_scene = q->r.scene;

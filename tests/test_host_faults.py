@@ -39,3 +39,11 @@ def test_batch_download_into_shared_buffers_and_after_faults(tmp_path):
                 ["engine.cpp", "image.cpp", "capi.cpp", "batch.cpp"])
     run(exe, "shared")
     print(run(exe, "faults"))
+
+
+def test_server_after_a_failed_request(tmp_path):
+    """Whichever call of a served request fails, the requests after it get
+    their own scenes' frames."""
+    exe = build(tmp_path, "serve_faults",
+                ["engine.cpp", "image.cpp", "capi.cpp", "serve.cpp"])
+    print(run(exe))
