@@ -281,8 +281,9 @@ int  qrhip_batch_tune(qrhip_batch *b, int reps, int *best, float *ms);
  * takes, within a budget of camera samples, a chunk of the oldest request in
  * flight and then chunks of the requests with the least work left, traces
  * the Whitted chunks as one batch (one launch per pipeline stage) and a
- * pass of each path-traced chunk (without a time budget, as many passes as
- * the step's samples allow), and returns the frames that finished.
+ * pass of each path-traced chunk (more, where that keeps the step within its
+ * time budget or, without one, within 2^22 samples), and returns the frames
+ * that finished.
  * Steps are pipelined (the next is launched before the last is retired).
  * Requests that arrive during a step join the next one, so a small frame
  * does not wait for a large one to finish.  A frame is the same whatever
@@ -334,7 +335,7 @@ typedef struct qrhip_server_stats
 /* scenes must be updated, on dev, and left to the server until it is
  * destroyed; hbm_budget bounds the summed footprint of requests in flight;
  * max_active bounds the requests in flight; step_samples is the camera
- * samples (path-traced samples count twice) a step takes, 0 for whole frames
+ * samples a step takes, 0 for whole frames
  * (max_active 1 and step_samples 0: one frame at a time, unbatched) */
 int  qrhip_server_create(qrhip_dev *dev, qrhip_scene *const *scenes, int n_scenes,
                          uint64_t hbm_budget, int max_active, uint64_t step_samples,
@@ -344,7 +345,9 @@ int  qrhip_server_submit(qrhip_server *s, const qrhip_request *req);
 /* completed requests, up to max, waiting up to wait_ms for the first one;
  * returns how many were written */
 int  qrhip_server_poll(qrhip_server *s, qrhip_result *out, int max, int wait_ms);
-/* device memory a request needs while in flight, in bytes */
+/* device memory a request needs while in flight, in bytes: its frame, tables,
+ * planes and the queues of its chunks (a path-traced request that exceeds the
+ * budget by its queues alone is accepted, and served by itself) */
 int  qrhip_server_footprint(qrhip_server *s, const qrhip_request *req, uint64_t *bytes);
 int  qrhip_server_get_stats(qrhip_server *s, qrhip_server_stats *st);
 /* a step's budget of predicted device time in ms (0, the default: only the

@@ -15,7 +15,8 @@
  * estimated device time and a cap of camera samples; it traces its Whitted
  * chunks as one batch of the level pipeline (one launch per stage for all
  * of them) and one run of passes of each path-traced chunk (as many passes
- * as the budget leaves room for).  The estimate is each scene's measured
+ * as the budget leaves room for; without a time budget one, and more only up
+ * to a few million samples in the whole step).  The estimate is each scene's measured
  * device time per sample, Whitted and path-traced apart: every retired step
  * times its Whitted batch and its path-traced runs with events and scales
  * the rates of the scenes in it by measured over predicted.
@@ -76,6 +77,7 @@ struct Req
 {
     qrhip_request r;
     uint64_t      bytes = 0;
+    uint64_t      run_max = 0;          /* path tracer: samples of its largest run */
     int           slot = -1;
     int           steps = 0;
     int           chunks_left = 0;      /* chunks with passes not retired */
@@ -99,6 +101,18 @@ struct SceneState
  * path-traced run (reset, bounces, fold), in ms */
 constexpr double WHITTED_STEP_MS = 0.15;
 constexpr double PT_RUN_MS = 0.10;
+
+/* samples a step without a time budget takes when its path-traced chunks are
+ * given more than one pass each (2 ms of device time): longer runs fill the
+ * chip better, but a frame that arrives meanwhile waits for the step.  16
+ * requests at once, two of them path-traced at 1280x720 and 16 spp: 32.5 ms
+ * with one pass a step, 30.0 at 2^22 samples, 29.6 at 2^23, 28.0 at 2^24. */
+constexpr uint64_t PT_STEP_SAMPLES = 1ull << 22;
+/* bound of the runs of a server with a time budget, in samples per ms of it
+ * (the box at 1280x720 traces 2.1e6 in one) */
+constexpr double PT_SAMPLES_PER_MS = 4e6;
+/* qr_pt_launch splits longer runs */
+constexpr uint64_t PT_RUN_SAMPLES = 1ull << 25;
 
 /* one chunk of a step: a Whitted chunk, or npass passes of a path-traced
  * chunk from pass pts_c on */
@@ -127,14 +141,32 @@ struct StepCtx
 /* bytes of a scene's tables on the device */
 uint64_t tables_bytes(const qr_device_tables &t)
 {
-    return sizeof(qr_surface) * (uint64_t)t.n_surf + sizeof(qr_material) * (uint64_t)t.n_mat +
+    return (sizeof(qr_surface) + sizeof(qr_dev_surf)) * (uint64_t)t.n_surf + sizeof(qr_material) * (uint64_t)t.n_mat +
            sizeof(qr_light) * (uint64_t)t.n_lgt + sizeof(qr_clip) * (uint64_t)t.n_clip +
            sizeof(qr_elem) * (uint64_t)t.n_elem + 4 * (uint64_t)t.n_texel +
            sizeof(qr_dev_step) * (uint64_t)(t.n_step + t.n_step_any + 2) +
            (sizeof(qr_refit_elem) + 32) * (uint64_t)t.n_elem;
 }
 
-uint64_t footprint(const qrhip_request &r, const qr_device_tables &t, uint64_t step_samples)
+/* samples of the largest run of passes a path-traced request is given: one
+ * pass of its largest chunk, or as many as a step allows */
+uint64_t run_samples(const qrhip_request &r, uint64_t step_samples, double step_ms)
+{
+    if (r.spp == 0) return 0;
+    const uint64_t ns = r.fsaa == 2 ? 4 : r.fsaa == 1 ? 2 : 1;
+    const uint64_t per_tile = 64 * ns;
+    uint64_t tiles = qr_pt_tiles(r.x_res, r.y_res);
+    if (step_samples > 0) tiles = std::min(tiles, std::max<uint64_t>(1, step_samples / per_tile));
+    const uint64_t pass = tiles * per_tile;
+    uint64_t most = step_ms > 0.0 ? (uint64_t)std::min((double)PT_RUN_SAMPLES,
+                                                       step_ms * PT_SAMPLES_PER_MS)
+                                  : PT_STEP_SAMPLES;
+    if (step_samples > 0) most = std::min(most, step_samples);
+    return std::max(pass, std::min(pass * (uint64_t)r.spp, most));
+}
+
+/* device memory of a request without its path-traced runs' queues */
+uint64_t base_footprint(const qrhip_request &r, const qr_device_tables &t, uint64_t step_samples)
 {
     const int n_lgt = t.n_lgt;
     const uint64_t ns = r.fsaa == 2 ? 4 : r.fsaa == 1 ? 2 : 1;
@@ -148,6 +180,15 @@ uint64_t footprint(const qrhip_request &r, const qr_device_tables &t, uint64_t s
     b += (uint64_t)r.depth * (n0 / 8 + 256) * (9 * 16 + 4); /* deeper levels */
     b += n0 * (uint64_t)std::max(1, n_lgt) * 12;            /* shadow jobs, 3 sets */
     return b;
+}
+
+/* and with them: a chunk's runs alternate between the two steps in flight,
+ * each with queues of its own */
+uint64_t footprint(const qrhip_request &r, const qr_device_tables &t, uint64_t step_samples,
+                   double step_ms)
+{
+    const uint64_t b = base_footprint(r, t, step_samples);
+    return r.spp > 0 ? b + 2 * qr_pt_run_bytes(run_samples(r, step_samples, step_ms)) : b;
 }
 
 hipError_t pinned_reserve(uint32_t *&p, size_t &cap, size_t n)
@@ -313,8 +354,9 @@ hipError_t qrhip_server::admit_one(Req *q)
 /* the step's chunks: requests in order of their deadlines, each chunk
  * taken while the step's predicted device time stays within budget_ms (0:
  * no time budget) and its samples within the server's cap; a step takes at
- * least one chunk.  A path-traced chunk takes as many passes as the budget
- * leaves room for, and none while its last run is in flight. */
+ * least one chunk.  A path-traced chunk takes as many passes as the time
+ * budget leaves room for (without one, a pass and a share of what is left of
+ * a short step), and none while its last run is in flight. */
 void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
 {
     units.clear();
@@ -349,25 +391,20 @@ void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
                 break;      /* the rest of this request waits; others may fit */
             }
             int npass = 1;
-            if (pt)
+            if (pt && budget_ms > 0.0)
             {
                 const int left = ch.passes - ch.enqueued;
                 int by_time = left, by_cap = left;
-                if (budget_ms > 0.0 && pass_ms > 0.0)
+                if (pass_ms > 0.0)
                 {
                     by_time = (int)std::max(1.0, (budget_ms - used_ms - fixed) / pass_ms);
-                }
-                else if (cap == ~0ull)
-                {
-                    /* whole frames: as many passes as a run of 2^24 samples */
-                    by_time = (int)std::max<uint64_t>(1, std::min<uint64_t>(
-                        (uint64_t)left, (1ull << 24) / std::max<uint64_t>(1, ch.cost)));
                 }
                 if (cap != ~0ull)
                 {
                     by_cap = (int)std::max<uint64_t>(1, (cap - std::min(cap, used_s)) / ch.cost);
                 }
-                npass = std::max(1, std::min(left, std::min(by_time, by_cap)));
+                const int by_run = (int)std::min<uint64_t>((uint64_t)left, q->run_max / ch.cost);
+                npass = std::max(1, std::min(std::min(left, by_run), std::min(by_time, by_cap)));
             }
             const double est = fixed + pass_ms * npass;
             units.push_back(Unit{q, c, (float)(ch.enqueued + 1), npass, est});
@@ -377,6 +414,26 @@ void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
             any_whitted = any_whitted || !pt;
         }
         if ((budget_ms > 0.0 && used_ms >= budget_ms) || used_s >= cap) break;
+    }
+    if (budget_ms > 0.0) return;
+
+    /* no time budget: every chunk has its pass; what is left of a short step
+     * goes to the path-traced ones in equal shares */
+    const uint64_t lim = std::min(cap, PT_STEP_SAMPLES);
+    uint64_t n_pt = 0;
+    for (const Unit &u : units) n_pt += u.q->r.spp > 0;
+    for (Unit &u : units)
+    {
+        if (u.q->r.spp == 0) continue;
+        if (used_s >= lim) break;
+        Chunk &ch = u.q->chunks[u.c];
+        const uint64_t share = std::min((lim - used_s) / n_pt--, u.q->run_max - ch.cost);
+        const int more = (int)std::min<uint64_t>((uint64_t)(ch.passes - ch.enqueued),
+                                                 share / ch.cost);
+        u.npass += more;
+        u.est_ms += (double)ch.cost * more * scenes[u.q->r.scene].pt_ns * 1e-6;
+        ch.enqueued += more;
+        used_s += ch.cost * (uint64_t)more;
     }
 }
 
@@ -773,7 +830,8 @@ int qrhip_server_footprint(qrhip_server *s, const qrhip_request *req, uint64_t *
     if (s == nullptr || req == nullptr || bytes == nullptr) return fail(QRHIP_E_ARG, "null argument");
     if (req->scene < 0 || req->scene >= (int)s->scenes.size())
         return fail(QRHIP_E_ARG, "scene index out of range");
-    *bytes = footprint(*req, s->scenes[req->scene].s->dt.t, s->step_samples);
+    std::lock_guard<std::mutex> lk(s->mu);
+    *bytes = footprint(*req, s->scenes[req->scene].s->dt.t, s->step_samples, s->step_ms);
     return QRHIP_OK;
 }
 
@@ -791,14 +849,17 @@ int qrhip_server_submit(qrhip_server *s, const qrhip_request *req)
     Req *q = new (std::nothrow) Req();
     if (q == nullptr) return fail(QRHIP_E_DEVICE, "out of host memory");
     q->r = r;
-    q->bytes = footprint(r, s->scenes[r.scene].s->dt.t, s->step_samples);
-    if (q->bytes > s->budget)
+    const qr_device_tables &t = s->scenes[r.scene].s->dt.t;
+    if (base_footprint(r, t, s->step_samples) > s->budget)
     {
         delete q;
         return fail(QRHIP_E_ARG, "request needs more device memory than the server's budget");
     }
     {
         std::lock_guard<std::mutex> lk(s->mu);
+        /* (a request that fits but for its queues is served by itself) */
+        q->run_max = run_samples(r, s->step_samples, s->step_ms);
+        q->bytes = std::min(footprint(r, t, s->step_samples, s->step_ms), s->budget);
         if (s->stop)
         {
             delete q;

@@ -334,6 +334,9 @@ hipError_t qr_pt_launch(qr_pt_state *s, const qr_device_tables *t, const qr_fram
 int        qr_pt_check(qr_pt_state *s);
 hipError_t qr_pt_retry(qr_pt_state *s, hipStream_t stream);
 uint32_t   qr_pt_tiles(int x_res, int y_res);
+/* device memory of a state's queues for runs of up to "samples" samples
+ * (slots times passes; an overflowed queue grows beyond it) */
+uint64_t   qr_pt_run_bytes(uint64_t samples);
 
 /* level-by-level pipeline (tracer_wf.hip): queues and counters of one
  * device, reused by every frame traced with it */

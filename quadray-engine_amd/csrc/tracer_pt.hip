@@ -767,6 +767,13 @@ uint32_t qr_pt_tiles(int x_res, int y_res)
     return (uint32_t)((x_res + PT_TILE - 1) / PT_TILE) * (uint32_t)((y_res + PT_TILE - 1) / PT_TILE);
 }
 
+uint64_t qr_pt_run_bytes(uint64_t samples)
+{
+    /* two ray queues, the contributions and the list heads (pt_reserve) */
+    return 2 * (4 * 16 + 4) * (uint64_t)round_up(samples) +
+           (16 + 4) * (uint64_t)round_up(samples / 4 + 1024) + 4 * samples;
+}
+
 hipError_t qr_pt_start(float *planes, uint32_t *seeds, int x_res, int y_res, int x_row,
                        int fsaa, hipStream_t stream)
 {

@@ -97,6 +97,7 @@ hipError_t qr_pt_launch(qr_pt_state *, const qr_device_tables *t, const qr_frame
 int qr_pt_check(qr_pt_state *) { return 0; }
 hipError_t qr_pt_retry(qr_pt_state *, hipStream_t) { return hipSuccess; }
 uint32_t qr_pt_tiles(int x_res, int y_res) { return qr_wf_batch_tiles(nullptr, x_res, y_res); }
+uint64_t qr_pt_run_bytes(uint64_t samples) { return samples; }
 
 namespace qrhip_impl {
 hipError_t noalloc_setup(int) { return hipSuccess; }

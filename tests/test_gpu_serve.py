@@ -7,6 +7,7 @@ with set_pton (path tracer) -- also when the frame is traced in chunks of a
 few tiles over many steps beside other requests.  Admission keeps the
 requests in flight within the memory budget; requests arriving while others
 run join later steps."""
+import ctypes as C
 import threading
 import time
 
@@ -224,6 +225,75 @@ def test_serve_time_budget_and_one_scene_at_many_times(device):
             s.destroy()
             w.close()
         assert np.array_equal(got[r.tag], want), f"request {r.tag} vs its scene"
+
+
+def _device_bytes_free():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert qrhip.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("step_samples", [0, 1 << 24])
+def test_serve_path_traced_memory_and_steps(device, step_samples):
+    """Path-traced requests on a server without a time budget: what the
+    server allocates stays within the requests' footprints, a request takes
+    many steps, and a small frame submitted behind them does not wait for
+    them.  (64 passes of 640x360 are 3.5 times the samples a step gives to
+    path-traced chunks beyond a pass of each.)"""
+    print(f"case path-traced requests, step of {step_samples} samples", flush=True)
+    sc = Scenes(device, [(7, 701), (3, 702)])
+    reqs = [qrhip.Server.request(k, 1, 640, 360, 0, 6, spp=64) for k in range(6)]
+    small = qrhip.Server.request(6, 0, 96, 64, 1, 3)
+    srv = qrhip.Server(device, sc.scenes, 64 << 30, 64, step_samples)
+    try:
+        need = sum(srv.footprint(r) for r in reqs + [small])
+        free = _device_bytes_free()
+        frames = {r.tag: srv.submit(r) for r in reqs + [small]}
+        results = {}
+        deadline = time.time() + 60
+        while len(results) < 7 and time.time() < deadline:
+            results.update({r["tag"]: r for r in srv.poll(wait_ms=200)})
+        used = free - _device_bytes_free()
+        stats = srv.stats()
+    finally:
+        srv.destroy()
+    try:
+        assert len(results) == 7 and all(r["status"] == 0 for r in results.values())
+        # (allocations are rounded up to 2 MiB, some 20 buffers a request)
+        assert used <= need + 7 * 20 * (2 << 20), (used >> 20, need >> 20)
+        assert 0 < stats["bytes_peak"] <= need
+        assert min(results[k]["steps"] for k in range(6)) >= 4
+        assert results[6]["done_ms"] < min(results[k]["done_ms"] for k in range(6))
+        for r in (reqs[0], small):
+            one, _, _ = serve(device, sc.scenes, [r], max_active=1, step_samples=0)
+            assert np.array_equal(frames[r.tag], one[r.tag])
+        for r in reqs:
+            assert np.array_equal(frames[r.tag], frames[0])
+    finally:
+        sc.close()
+
+
+def test_serve_budget_below_the_queues(device):
+    """A budget that holds a path-traced request's planes but not its queues
+    serves such requests one at a time; one that does not hold the planes
+    refuses them."""
+    sc = Scenes(device, [(3, 703)])
+    try:
+        reqs = [qrhip.Server.request(k, 0, 96, 64, 0, 6, spp=3) for k in range(3)]
+        got, _, stats = serve(device, sc.scenes, reqs, budget=1 << 20)
+        assert stats["step_frames_max"] == 1 and stats["bytes_peak"] <= 1 << 20
+        free, _, _ = serve(device, sc.scenes, reqs)
+        for r in reqs:
+            assert np.array_equal(got[r.tag], free[r.tag])
+        srv = qrhip.Server(device, sc.scenes, 1 << 16, 8, CHUNK)
+        try:
+            assert srv.footprint(reqs[0]) > 1 << 20
+            with pytest.raises(qrhip.QrError, match="device memory"):
+                srv.submit(reqs[0])
+        finally:
+            srv.destroy()
+    finally:
+        sc.close()
 
 
 def test_serve_rejects_bad_requests(device):
