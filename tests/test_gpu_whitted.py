@@ -6,6 +6,8 @@ kernels meet with every pixel identical (they apply QuadRay's operations in
 its order), so frames are required bit-identical; first-hit ids identical
 except on rays the oracle flags as near-zero discriminant (|D| < 1e-5, where
 fp32 root selection is ill-conditioned)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -450,6 +452,38 @@ def test_gpu_frames_without_secondary_rays(path_dev, config, x, y, fsaa, depth):
         hs.close()
     assert_frame_exact(got, want, "frame")
     assert not np.any((gid != wid) & (flags == 0))
+
+
+def test_gpu_scene_creation_waits_for_no_other_work(device):
+    """A scene with a frame of its own is made, blank, while the program's
+    default stream is busy, or the device's own."""
+    rt, n = qrhip.lib(), 1 << 31
+    buf = C.c_void_p()
+    assert rt.hipMalloc(C.byref(buf), C.c_size_t(n)) == 0
+    works = [qrhip.Workload(2, 54 + k) for k in range(3)]
+    scenes = [qrhip.Scene(device, works[0].ptr, 1920, 1080)]
+    try:
+        scenes[0].set_depth(8)
+        scenes[0].render(0)
+        assert rt.hipMemset(buf, 0, C.c_size_t(n)) == 0
+        for _ in range(100):            # tens of milliseconds
+            assert rt.hipMemsetAsync(buf, 0, C.c_size_t(n), None) == 0
+        scenes.append(qrhip.Scene(device, works[1].ptr, 1281, 719))
+        busy = rt.hipStreamQuery(None)
+        assert not scenes[1].frame().any()
+        assert rt.hipDeviceSynchronize() == 0
+        for _ in range(20):
+            qrhip.check(rt.qrhip_scene_launch(scenes[0].h))
+        scenes.append(qrhip.Scene(device, works[2].ptr, 1281, 719))
+        assert not scenes[2].frame().any()
+        qrhip.check(rt.qrhip_scene_sync(scenes[0].h))
+    finally:
+        assert rt.hipFree(buf) == 0
+        for s in scenes:
+            s.destroy()
+        for w in works:
+            w.close()
+    assert busy == 600      # hipErrorNotReady: the fills were still running
 
 
 def test_gpu_depth_changes_path_between_frames(device):
