@@ -121,7 +121,6 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
     Node stk[MAX_STACK];
     int sp = 0;
     V3 ret = {0.0f, 0.0f, 0.0f};
-    bool primary = true;
 
     for (;;)
     {
@@ -131,11 +130,11 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
         if (!walk<false>(sc, ray, h))
         {
             ret = V3{0.0f, 0.0f, 0.0f};
-            if (primary) *hit_id = -1;
+            if (ray.origin < 0) *hit_id = -1;       /* (the camera's ray) */
         }
         else
         {
-            if (primary) *hit_id = (sc.srf[h.srf].id << 1) | h.side;
+            if (ray.origin < 0) *hit_id = (sc.srf[h.srf].id << 1) | h.side;
             hit_info(sc, ray, h);
             const V3 nrm = normal_at(sc, h);
             Node &nd = stk[sp];
@@ -158,7 +157,6 @@ __device__ V3 trace_sample(const Scene &sc, const qr_frame_desc &fd, Ray ray,
                 ret = nd.col;
             }
         }
-        primary = false;
         if (descend)
         {
             sp++;
