@@ -562,6 +562,15 @@ __device__ __forceinline__ void roots_mid(float a_val, float b_val, float c_val,
     q.d2 = x ? qq : a_val;
 }
 
+/* the next float above t_lim; 0 for one below zero (a kept distance of a ray
+ * whose t_min is), which turns away no root the limit allows */
+template <bool T0>
+__device__ __forceinline__ float above(float t_lim)
+{
+    const int32_t next = (int32_t)(fbits(t_lim) + 1u);
+    return bitsf((uint32_t)(T0 || next > 0 ? next : 0));
+}
+
 /* the lanes whose n / d, rounded, may lie above t_min and at or below
  * t_lim, given the next float above t_lim; never without one that does.  With n'
  * = n times the sign of d and d' = |d|: rounding is monotonic and t_min a
@@ -859,7 +868,7 @@ __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
                 }
                 if (keep != 0)
                 {
-                    const float t_next = bitsf(fbits(t_lim) + 1u);
+                    const float t_next = above<T0>(t_lim);
                     /* the lanes with a first and a second root, and those
                      * whose first is of side 1 */
                     uint64_t m1, m2 = 0, side, dmask = 0;

@@ -410,6 +410,40 @@ def test_gpu_world_surfaces_in_a_group(path_dev, config, depth):
         assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
 
 
+@pytest.mark.parametrize("config,depth", [(1, 0), (1, 3), (9, 0), (9, 3)])
+@pytest.mark.parametrize("back", [False, True])
+def test_gpu_equal_distances(path_dev, config, depth, back):
+    """Coincident surfaces, whose roots are equal: the later one of the list
+    is seen, also at distances below zero ("back": a camera turned away, with
+    a near clip behind it); bit for bit the oracle's frame."""
+    snap = _snapshot(config, 23, 95, 61, 1, depth)
+    t = qrhip.TablesFromSnapshot(snap)
+    t.tables.n_step = t.tables.n_step_any = 0
+    world = [i for i in range(t.tables.n_surf)
+             if t.tables.surfaces[i].tag >= 0 and t.tables.surfaces[i].shift == 0]
+    assert len(world) >= 5
+    for a, b in zip(world[0::2], world[1::2]):
+        keep = {k: list(getattr(t.tables.surfaces[b], k)) for k in ("mat", "props")}
+        own = t.tables.surfaces[b].id
+        C.memmove(C.byref(t.tables.surfaces[b]), C.byref(t.tables.surfaces[a]),
+                  C.sizeof(qrhip.QrSurface))
+        t.tables.surfaces[b].id = own
+        for k, v in keep.items():
+            for side in range(2):
+                getattr(t.tables.surfaces[b], k)[side] = v[side]
+    if back:
+        t.fd.t_min = -1.0e30
+        for field in ("dir", "hor", "ver"):
+            v = getattr(t.fd, field)
+            for k in range(len(v)):
+                v[k] = -v[k]
+    want, ids_o, flags, _, _ = qr_oracle.render(t.ptr, t.fd, want_ids=True)
+    assert (ids_o >= 0).any()
+    for got, ids in _render_every_way(path_dev, t):
+        assert_frame_exact(got, want, f"config {config} depth {depth} back {back}")
+        assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
+
+
 @pytest.mark.parametrize("config,x,y,fsaa,depth", [
     # 16 lanes to a sample: the smallest frame, ragged edges of every tile
     # shape, the largest number of samples; then 4, 2 and 1 lanes
