@@ -134,12 +134,14 @@ static inline QR_HD void qr_dev_surf_of(const qr_surface *r, int n_surf, qr_dev_
         }
         if (pure) f = unit ? QR_DC_SPHERE : QR_DC_PURE;
     }
+    const uint32_t cls = f;
     if (r->shift != 0) f |= QR_DS_SHIFT;
     const uint32_t trm = r->trm == 0 ? 0u : r->trm == 1 ? QR_DI_TRM_DIAG
                                           : r->trm == 2 ? QR_DI_TRM_ROT : QR_DI_TRM;
     if (r->shift != 0 || r->tag < 0) f |= trm * QR_DS_TRM_DIAG;
     if (r->shift == 0 || r->tag < 0) f |= QR_DS_SOLO;
-    if (r->apex != 0) f |= QR_DS_APEX;
+    /* (a plane has no apex, whatever its record says) */
+    if (r->apex != 0 && cls != QR_DC_PLANE) f |= QR_DS_APEX;
     if (r->apex == 2) f |= QR_DS_APEX_TWO;
     f |= ((uint32_t)r->cmin_on & 7u) << QR_DS_CMIN_BIT;
     f |= ((uint32_t)r->cmax_on & 7u) << QR_DS_CMAX_BIT;

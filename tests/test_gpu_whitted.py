@@ -410,6 +410,21 @@ def test_gpu_world_surfaces_in_a_group(path_dev, config, depth):
         assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
 
 
+@pytest.mark.parametrize("config,depth", [(1, 2), (9, 2), (2, 2)])
+def test_gpu_planes_have_no_apex(path_dev, config, depth):
+    """An apex kind in a plane's record changes nothing, whatever its
+    thresholds: bit for bit the oracle's frame."""
+    t = qrhip.TablesFromSnapshot(_snapshot(config, 25, 95, 61, 1, depth))
+    for i in range(t.tables.n_surf):
+        s = t.tables.surfaces[i]
+        if s.solver == 1:
+            s.apex, s.d_eps, s.t_eps = 1 + i % 2, 1.0e6, 1.0e6
+    want, ids_o, flags, _, _ = qr_oracle.render(t.ptr, t.fd, want_ids=True)
+    for got, ids in _render_every_way(path_dev, t):
+        assert_frame_exact(got, want, f"config {config}")
+        assert np.array_equal(ids[flags == 0], ids_o[flags == 0])
+
+
 @pytest.mark.parametrize("config,depth", [(1, 0), (1, 3), (9, 0), (9, 3)])
 @pytest.mark.parametrize("back", [False, True])
 def test_gpu_equal_distances(path_dev, config, depth, back):
