@@ -344,3 +344,24 @@ def test_batch_with_and_without_secondary_rays(device):
             hs.close()
         assert np.array_equal(frame, want), f"batched frame {key}"
         assert np.array_equal(alone(device, *key), want), f"frame {key} alone"
+
+
+@pytest.mark.parametrize("config,depth", [(1, 4), (2, 0), (4, 0), (9, 0)])
+def test_one_frame_batch_without_secondary_rays(device, config, depth):
+    """A batch of one frame traces its single level through the pipeline's
+    queues (alone, most such frames are one kernel): ragged sizes at 1, 2
+    and 4 samples, direct, as a graph and serially, against the oracle."""
+    for x, y, fsaa in ((1, 1, 2), (67, 35, 0), (131, 77, 1), (93, 61, 2), (259, 3, 1)):
+        bc = BatchCase(device, [(config, 26)], [(0, x, y, fsaa, depth)])
+        try:
+            got = [bc.batch.render(mode)[0].copy()
+                   for mode in (qrhip.BATCH_DIRECT, qrhip.BATCH_GRAPH, qrhip.BATCH_SERIAL)]
+        finally:
+            bc.close()
+        hs = HostScene(config, 26, x, y, fsaa, depth)
+        try:
+            want = hs.oracle()[0]
+        finally:
+            hs.close()
+        for frame in got:
+            assert np.array_equal(frame, want), (config, x, y, fsaa)

@@ -471,18 +471,24 @@ def test_gpu_equal_distances(path_dev, config, depth, back):
 ])
 def test_gpu_one_kernel_lanes_per_sample(device, config, x, y, fsaa, depth):
     """However many lanes trace a sample, and over ragged tiles, the frame and
-    the first-hit ids are those of the level pipeline."""
+    the first-hit ids are those of the level pipeline, or of the oracle where
+    a frame without secondary rays would take the one kernel on both paths."""
     device.set_fsaa(fsaa)
     hs = HostScene(config, 51, x, y, fsaa, depth)
     try:
-        want, wid = device.render_tables(hs.tables, hs.fd, want_ids=True)
+        same = np.ones(1, dtype=bool)
+        if config == 1 or depth == 0:
+            want, wid, flags, _, _ = hs.oracle(want_ids=True)
+            same = flags == 0
+        else:
+            want, wid = device.render_tables(hs.tables, hs.fd, want_ids=True)
         device.set_path(qrhip.PATH_ONE_KERNEL)
         got, gid = device.render_tables(hs.tables, hs.fd, want_ids=True)
     finally:
         device.set_path(qrhip.PATH_LEVELS)
         hs.close()
     assert np.array_equal(got, want)
-    assert np.array_equal(gid, wid)
+    assert not np.any((gid != wid) & same)
 
 
 @pytest.mark.parametrize("config,x,y,fsaa,depth", [
