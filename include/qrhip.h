@@ -164,7 +164,8 @@ int  qrhip_render_tables(qrhip_dev *dev, const qr_scene_tables *tables,
  * one-kernel path; every device buffer it needs beyond the caller's host
  * inputs and outputs (staged tables, culling programs, device frame and ids)
  * comes from one static device array of QRHIP_NOALLOC_BYTES per GPU, held
- * until the process ends.  It calls no device allocator; tables plus frame
+ * until the process ends, and the walks' form of the surfaces from a second
+ * one of 39 MiB, sized so that it refuses nothing the first holds.  It calls no device allocator; tables plus frame
  * (4 bytes a pixel) plus ids (4 bytes a sample) beyond that size are
  * rejected with QRHIP_E_ARG, and so is a row pitch shorter than a row.
  * Calls that overlap on one GPU share the array and race: serialise them. */

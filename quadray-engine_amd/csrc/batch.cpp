@@ -277,7 +277,7 @@ hipError_t finish(qrhip_batch *b)
 
 /* capture the direct launch sequence in a graph; the frame arguments and
  * queues are settled by a direct run first, so the captured launches only
- * enqueue kernels and the counter copy */
+ * enqueue kernels (the resolve writes the counters to the host) */
 hipError_t capture(qrhip_batch *b)
 {
     hipError_t e;

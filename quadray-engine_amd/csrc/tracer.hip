@@ -65,7 +65,7 @@ __device__ __forceinline__ V3 hit_colour(const Scene &sc, const qr_frame_desc &f
     V3 col = shade_base(sc, fd, h, tex, lit);
     for (int l0 = 0; lit && l0 < sc.n_lgt; l0 += SPLIT)
     {
-        /* this lane's light of the next four, then all four added in
+        /* this lane's light of the next SPLIT, then all of them added in
          * their order */
         const int li = l0 + sub;
         Ray sr;
@@ -82,10 +82,10 @@ __device__ __forceinline__ V3 hit_colour(const Scene &sc, const qr_frame_desc &f
             Hit sh;
             vis = !walk<true>(sc, sr, sh);
         }
-        const uint32_t four = (uint32_t)(lanes(vis) >> group);
+        const uint32_t seen = (uint32_t)(lanes(vis) >> group);
         for (int k = 0; k < SPLIT && l0 + k < sc.n_lgt; k++)
         {
-            if (!((four >> k) & 1u)) continue;
+            if (!((seen >> k) & 1u)) continue;
             const QC qr_light &l = sc.lgt[l0 + k];
             V3 L;
             const float dot = light_vec(l, h.hit, nrm, L);

@@ -69,8 +69,8 @@ __device__ __forceinline__ bool all_mid(float x)
 /* sqrtf(x) and 1.0f / sqrtf(x), both roundings as they are: the short forms
  * where the whole wave's values are in sqrt_mid's range (nearly always).
  * There the root is in [2^-48, 2^64), and the hardware reciprocal with one
- * Newton step is the correctly rounded reciprocal (compared with 1.0f /
- * sqrtf(x) on every float of the range).  12 VALU instructions and the test
+ * Newton step is the correctly rounded reciprocal (tests/test_gpu_math.py
+ * compares every float).  12 VALU instructions and the test
  * instead of 27. */
 __device__ __forceinline__ float root(float x)
 {
@@ -182,14 +182,14 @@ struct Hit
     float u, v;
 };
 
-/* inverse-matrix product, diagonal first (tracer.cpp:2536-2568); td its
- * diagonal, to the rest */
 template <class P>
 __device__ __forceinline__ V3 sub3(const V3 &a, P p)
 {
     return V3{a.x - p[0], a.y - p[1], a.z - p[2]};
 }
 
+/* inverse-matrix product, diagonal first (tracer.cpp:2536-2568); td its
+ * diagonal, to the rest */
 __device__ __forceinline__ V3 xform_full(const float td[3], const float to[6], const V3 &d)
 {
     V3 o;
@@ -594,17 +594,6 @@ __device__ __forceinline__ float slab_rcp(float d)
     return fminf(fmaxf(__builtin_amdgcn_rcpf(d), -1e30f), 1e30f);
 }
 
-/* does any active lane of the wave hold b (the lane mask stays in scalar
- * registers) */
-__device__ __forceinline__ bool wave_any(bool b)
-{
-    return __builtin_amdgcn_ballot_w64(b) != 0;
-}
-
-/* a ray's side of the box tests: its clamped reciprocal direction and, per
- * axis, the offsets that place a box's bounds on the ray, with the ray's
- * share of the allowance (QR_CULL_FUZZ times the L1 distance of its origin
- * o from the boxes' reference point) moving each bound outwards */
 /* the step at byte offset "off" of a culling program (wave-uniform: one
  * 32-byte scalar load) */
 __device__ __forceinline__ qr_dev_step step_at(const QC qr_dev_step *prog, uint32_t off)
@@ -614,6 +603,10 @@ __device__ __forceinline__ qr_dev_step step_at(const QC qr_dev_step *prog, uint3
     return v;
 }
 
+/* a ray's side of the box tests: its clamped reciprocal direction and, per
+ * axis, the offsets that place a box's bounds on the ray, with the ray's
+ * share of the allowance (QR_CULL_FUZZ times the L1 distance of its origin
+ * o from the boxes' reference point) moving each bound outwards */
 struct BoxRay
 {
     float ix, iy, iz;
@@ -692,17 +685,13 @@ __device__ __forceinline__ bool own_list(const Scene &sc, int surf)
  * wave masks: no branch of the element work changes the active lanes, but
  * for the rare near-zero discriminants and apexes.
  *
- * What bounds it is VALU issue (the path tracer's bounces issue a VALU
- * instruction in 92% of their quad cycles), so a quadric takes only what its
- * class needs, its quotients are formed only for roots that can lie in the
- * ray's range, and a hit point only where the surface clips.  Against one
- * division per root and one clipping stage per root for every surface, read
- * from the 208-byte record: the bounces of a 1280x720 64-spp frame issue
- * 1.77e10 wave-level VALU instructions instead of 2.09e10, and 6.5e8 scalar
- * loads instead of 2.2e9 (the frame 37.5 -> 31.4 ms); a 641x359 4X frame of
- * glass 2.51 -> 2.21 ms, a 1080p 4X frame of 64 quadrics 2.11 -> 2.06 ms with
- * its copy to the host.  One body for both roots also makes the walks' code
- * a third shorter. */
+ * What bounds it is VALU issue (the path tracer's bounces are busy with it
+ * nine tenths of their time), so a quadric takes only what its class needs,
+ * its quotients are formed only for roots that can lie in the ray's range,
+ * and a hit point only where the surface clips: 1.77e10 wave-level VALU
+ * instructions and 6.5e8 scalar loads in the bounces of a 1280x720 64-spp
+ * frame, 2.09e10 and 2.2e9 with a division and a clipping stage per root read
+ * from the 208-byte record (37.5 -> 31.4 ms). */
 template <bool SHADOW, bool T0 = SHADOW>
 __device__ bool walk(const Scene &sc, const Ray &r, Hit &best, bool rev = true)
 {

@@ -230,7 +230,7 @@ __device__ __forceinline__ void put_ray(const PtArgs &a, int out, uint32_t idx, 
  * into queue L + 1 (3420-3920 emission, roulette and diffuse bounce;
  * 4686-4752 the refraction / reflection pick; 4762-4800, 5175-5215 their
  * throughputs) */
-/* six waves per SIMD (80 VGPRs, 32 bytes spilled): with workgroups handed out as
+/* six waves per SIMD (80 VGPRs, 36 bytes spilled): with workgroups handed out as
  * others finish, more resident waves hide more of the walks' latency
  * (measured per frame: 40.1 ms at five, 37.6 at six, 37.5 at seven with 34
  * spilled, 40.8 at eight) */

@@ -785,7 +785,7 @@ __global__ void __launch_bounds__(WG) k_shading(Batch b)
 /* a stage of two or three kinds of work: per frame, the shadow walks of
  * level b.sl, then the nearest walks of level b.wl >= 1, then the shading of
  * level b.fl >= 1 (shadow walks first measured 1.7% faster per frame) */
-/* seven waves per SIMD (72 VGPRs, 40 bytes spilled): the deeper levels' short
+/* seven waves per SIMD (72 VGPRs, 44 bytes spilled): the deeper levels' short
  * queues are latency bound (measured per frame: 1.775 ms at seven, 1.816
  * at six, 1.807 at eight with 29 spilled; five was 4% slower than six) */
 template <int R>
