@@ -106,7 +106,8 @@ constexpr double PT_RUN_MS = 0.10;
  * given more than one pass each (2 ms of device time): longer runs fill the
  * chip better, but a frame that arrives meanwhile waits for the step.  16
  * requests at once, two of them path-traced at 1280x720 and 16 spp: 32.5 ms
- * with one pass a step, 30.0 at 2^22 samples, 29.6 at 2^23, 28.0 at 2^24. */
+ * with one pass a step, 30.0 at 2^22 samples, 29.6 at 2^23, 28.0 at 2^24 (all
+ * path-traced chunks in one step; 29.2 at 2^22 with half of them in each). */
 constexpr uint64_t PT_STEP_SAMPLES = 1ull << 22;
 /* bound of the runs of a server with a time budget, in samples per ms of it
  * (the box at 1280x720 traces 2.1e6 in one) */
@@ -369,6 +370,15 @@ void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
     std::stable_sort(order.begin(), order.end(), [](const Req *x, const Req *y) {
         return x->deadline_ms < y->deadline_ms;
     });
+    /* a path-traced chunk in flight takes no run in the next step, so without
+     * a time budget half of them go into each: the device then has the next
+     * step's runs behind this one's */
+    size_t pt_room = 0;
+    for (const Req *q : active)
+    {
+        for (const Chunk &ch : q->chunks) pt_room += q->r.spp > 0 && ch.finished != ch.passes;
+    }
+    pt_room = budget_ms > 0.0 ? pt_room : (pt_room + 1) / 2;
     for (Req *q : order)
     {
         const bool pt = q->r.spp > 0;
@@ -381,7 +391,7 @@ void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
             /* a path-traced chunk's next pass reads the planes its last pass
              * writes, and a run that overflowed its queues is traced again
              * when its step retires: one run of a chunk in flight at a time */
-            if (pt && ch.enqueued != ch.finished) continue;
+            if (pt && (ch.enqueued != ch.finished || pt_room == 0)) continue;
             const double pass_ms = (double)ch.cost * ns_per * 1e-6;
             const double fixed = pt ? PT_RUN_MS : any_whitted ? 0.0 : WHITTED_STEP_MS;
             if (!units.empty() &&
@@ -412,13 +422,14 @@ void qrhip_server::pick(std::vector<Unit> &units, double budget_ms)
             used_ms += est;
             used_s += ch.cost * (uint64_t)npass;
             any_whitted = any_whitted || !pt;
+            pt_room -= pt ? 1 : 0;
         }
         if ((budget_ms > 0.0 && used_ms >= budget_ms) || used_s >= cap) break;
     }
     if (budget_ms > 0.0) return;
 
-    /* no time budget: every chunk has its pass; what is left of a short step
-     * goes to the path-traced ones in equal shares */
+    /* no time budget: every chunk of the step has its pass; what is left of a
+     * short step goes to the path-traced ones in equal shares */
     const uint64_t lim = std::min(cap, PT_STEP_SAMPLES);
     uint64_t n_pt = 0;
     for (const Unit &u : units) n_pt += u.q->r.spp > 0;
