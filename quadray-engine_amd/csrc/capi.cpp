@@ -499,12 +499,16 @@ int qrhip_scene_program_stats(qrhip_scene *s, int *builds, int *refits, int *mis
             if (memcmp(&got[(size_t)p], &want[(size_t)p], sizeof(qr_dev_step)) != 0) (*mismatch)++;
         }
     }
-    /* the records and materials (the device update stage writes them) */
+    /* the records, as they are and as the walks read them, and the materials
+     * (the device update stage writes them) */
     std::vector<qr_surface> srf((size_t)h.n_surf);
+    std::vector<qr_dev_surf> hot((size_t)h.n_surf);
     std::vector<qr_material> mat((size_t)h.n_mat);
     if (h.n_surf > 0)
     {
         HIP_TRY(hipMemcpy(srf.data(), s->dt.srf.ptr, sizeof(qr_surface) * srf.size(),
+                          hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpy(hot.data(), s->dt.hot.ptr, sizeof(qr_dev_surf) * hot.size(),
                           hipMemcpyDeviceToHost));
     }
     if (h.n_mat > 0)
@@ -515,6 +519,9 @@ int qrhip_scene_program_stats(qrhip_scene *s, int *builds, int *refits, int *mis
     for (int r = 0; r < h.n_surf; r++)
     {
         if (memcmp(&srf[(size_t)r], &h.surfaces[r], sizeof(qr_surface)) != 0) (*mismatch)++;
+        qr_dev_surf want;
+        qr_dev_surf_of(&h.surfaces[r], h.n_surf, &want);
+        if (memcmp(&hot[(size_t)r], &want, sizeof(want)) != 0) (*mismatch)++;
     }
     for (int m = 0; m < h.n_mat; m++)
     {
